@@ -454,203 +454,358 @@ __global__ __launch_bounds__(1024) void k_ktab(GridDev<T> g, int ntiles, T thr2,
 //   operator launch (A.op = 1): aw_out <- A W (TA, [v][K])
 //   per-solve mode 0 (term):  W <- g^l mu_s A W, dE = exitance(A W), bsum = stop-rule sums of W
 //   per-solve mode 2 (final): dE only
-// grid = (ceil(N/64), nsolve), block = 64.
-// ---------------------------------------------------------------------------
-template <typename T, typename TA, int L>
-__device__ __forceinline__ void combine_out(const CombArgs<T, TA> &A, const SolveDev<T, TA> &S, int v,
-                                            const TA (&acc)[(L + 1) * (L + 1)], const TA *__restrict__ wsum);
-
-
-template <typename T, typename TA, int L>
-__global__ __launch_bounds__(kWave) void k_combine(CombArgs<T, TA> A, const SolveDev<T, TA> *__restrict__ sv)
-{
-    constexpr int K = (L + 1) * (L + 1);
-    const GridDev<T> &g = A.g;
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    const SolveDev<T, TA> S = sv[blockIdx.y];
-    if (v >= g.N) return;
-    TA acc[K], w[K];
-#pragma unroll
-    for (int a = 0; a < K; ++a) {
-        acc[a] = TA(0);
-        w[a] = TA(S.W[(size_t)v * K + a]) / A.nsc[a];
-    }
-    for (int c = 0; c < A.nchunk; ++c) {
-        const T *__restrict__ p = S.part + ((size_t)c * g.N + v) * K;
-#pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] += TA(p[a]);
-    }
-    zpow_to_harmonic<TA, L>(acc);
-#pragma unroll
-    for (int a = 0; a < K; ++a) acc[a] *= A.nsc[a];
-    // self block: sum_k coef_k (M_k w), coef_k = (-mu)^{k-1}/k!
-    if constexpr (sizeof(T) == 4) {
-        // in FP32, on the entries the voxel's reflection symmetries leave
-        T wt[K], st[K];
-#pragma unroll
-        for (int a = 0; a < K; ++a) {
-            wt[a] = T(w[a]);
-            st[a] = T(0);
-        }
-        const T mu = S.mut[v];
-        T coef = T(1);
-        for (int k = 0; k < kNMom; ++k) {
-            if (k > 0) coef = coef * (-mu) / T(k + 1);
-            self_apply<K>(st, coef, A.momT + (size_t)k * K * K, wt, std::make_integer_sequence<int, K>{});
-        }
-#pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] += A.self_scale * TA(st[a]);
-    } else {
-        const TA mu = TA(S.mut[v]);
-        TA coef = TA(1);
-        for (int k = 0; k < kNMom; ++k) {
-            if (k > 0) coef = coef * (-mu) / TA(k + 1);
-            const TA *__restrict__ M = A.mom + (size_t)k * K * K;
-#pragma unroll
-            for (int a = 0; a < K; ++a) {
-                TA s = TA(0);
-#pragma unroll
-                for (int b = 0; b < K; ++b) s += M[a * K + b] * w[b];
-                acc[a] += A.self_scale * coef * s;
-            }
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < K; ++a) acc[a] *= A.dV;
-    if (A.op) {
-#pragma unroll
-        for (int a = 0; a < K; ++a) A.aw_out[(size_t)v * K + a] = acc[a];
-        return;
-    }
-    combine_out<T, TA, L>(A, S, v, acc, A.wsum);
-}
-
-// The per-solve outputs of one voxel's A W (acc, unscaled, TA): stored or
-// accumulated copies, the exitance and reflectance increments, and in a term
-// the scattered next term with its stop-rule sums (weights wsum).
-template <typename T, typename TA, int L>
-__device__ __forceinline__ void combine_out(const CombArgs<T, TA> &A, const SolveDev<T, TA> &S, int v,
-                                            const TA (&acc)[(L + 1) * (L + 1)], const TA *__restrict__ wsum)
-{
-    constexpr int K = (L + 1) * (L + 1);
-    const GridDev<T> &g = A.g;
-    const int zk = v / (g.nx * g.ny);
-    const int pix = v - zk * g.nx * g.ny;
-    const bool bottom = (zk == g.nz - 1);
-    if (S.aw_store) {
-#pragma unroll
-        for (int a = 0; a < K; ++a) S.aw_store[(size_t)v * K + a] = acc[a];
-    }
-    if (S.phi && S.mode != 3) {
-#pragma unroll
-        for (int a = 0; a < K; ++a) S.phi[(size_t)v * K + a] += acc[a];
-    }
-    if (bottom && S.mode != 3) {
-        TA e = TA(0);
-#pragma unroll
-        for (int l = 0; l <= L; ++l) e += A.coefE[l] * acc[l * l + l];
-        S.dE[pix] = e;
-    }
-    if (zk == 0 && S.mode != 3) {
-        TA r = TA(0);
-#pragma unroll
-        for (int l = 0; l <= L; ++l) r += A.coefR[l] * acc[l * l + l];
-        S.dR[pix] = r;
-    }
-    if (S.mode == 0 || S.mode == 3) {
-        const TA ms = TA(S.mus[v]);
-        TA gl = TA(1), bs = TA(0);
-#pragma unroll
-        for (int l = 0; l <= L; ++l) {
-#pragma unroll
-            for (int m = -l; m <= l; ++m) {
-                const int a = l * l + l + m;
-                const TA wn = gl * ms * acc[a];
-                const T wt = T(wn * A.nsc[a]);
-                S.W[(size_t)v * K + a] = wt;
-                bs += wsum[a] * (TA(wt) / A.nsc[a]);
-            }
-            gl *= TA(S.g);
-        }
-        if (bottom && S.mode == 0) S.bsum[pix] = bs;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Combine of frequency-domain solves: halves (sv[2y], sv[2y+1]) = (real,
-// imaginary) of one complex field.  The self block has the complex series
+// NH = 2: the solves (sv[2y], sv[2y+1]) are the (real, imaginary) halves of one
+// frequency-domain field.  The self block then has the complex series
 // coefficients c_k = (-mu)^{k-1}/k!, mu = mu_t + i kim:
 //   S (w0 + i w1) = sum_k (Re c_k M_k w0 - Im c_k M_k w1) + i (Re c_k M_k w1 + Im c_k M_k w0);
 // everything else acts on each half alone (D, the exitance and reflectance
-// functionals and the chunk sums are real).  Both halves' W are read before
-// either is overwritten by the scattered next term.
-// grid = (ceil(N/64), ncomplex), block = 64.
+// functionals and the chunk sums are real).  A block reads its voxels' W of all
+// halves before it overwrites any with the scattered next term.
+//
+// One thread per (voxel, coefficient), VPT voxels each: the chunk partials, W and
+// the outputs are read and written as runs of consecutive elements, and a grid of a
+// few thousand voxels fills the chip.  (One thread per voxel, the layout before
+// this, left 64 waves for 16^3 voxels, each with a chain of 64 chunks x 9 loads
+// and 16 moment matrices read through the scalar cache.)  Measured, L = 5, before ->
+// now: 16^3 159 -> 19 us, 32^3 106 -> 34 us (partials at 1.3 TB/s, latency), 64 solves of
+// 20^3 629 -> 377 us (2.5 GB of partials at 6.7 TB/s), FP64 14^3 593 -> 23 us; 8^3 at
+// L = 3 15.5 -> 7.1 us.  What a voxel's
+// coefficients exchange -- the z-power sums, W, the bottom sums -- goes through LDS.
+// FP32 self block: a coefficient couples to at most NJ others (self_couples), so
+// a thread keeps those NJ values of W and sums the moments' packed rows from LDS.
+// FP64 keeps all K (the couplings that symmetry makes ~1e-7, not 0): Y_k = M_k W
+// for 16 coefficients x 16 voxels on the FP64 matrix instruction, the moments read
+// once per tile instead of once per voxel.
+// grid = (ceil(N/VB), nsolve or ncomplex), block = kCombThreads.
 // ---------------------------------------------------------------------------
-template <typename T, typename TA, int L>
-__global__ __launch_bounds__(kWave) void k_combine_c(CombArgs<T, TA> A, const SolveDev<T, TA> *__restrict__ sv)
-{
-    constexpr int K = (L + 1) * (L + 1);
-    const GridDev<T> &g = A.g;
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    const SolveDev<T, TA> S0 = sv[2 * blockIdx.y], S1 = sv[2 * blockIdx.y + 1];
-    if (v >= g.N) return;
-    T w0[K], w1[K], st0[K], st1[K];
-#pragma unroll
-    for (int a = 0; a < K; ++a) {
-        w0[a] = T(TA(S0.W[(size_t)v * K + a]) / A.nsc[a]);
-        w1[a] = T(TA(S1.W[(size_t)v * K + a]) / A.nsc[a]);
-        st0[a] = st1[a] = T(0);
+constexpr int kCombThreads = 256;
+
+template <int L>
+struct CombShape {
+    static constexpr int K = (L + 1) * (L + 1);
+    static constexpr int VP = kCombThreads / K < 64 ? kCombThreads / K : 64;  // voxels side by side
+    static constexpr int VPT = 2;                                            // voxels per thread
+    static constexpr int VB = VP * VPT;
+    static constexpr int coupled(int a)
+    {
+        int c = 0;
+        for (int b = 0; b < K; ++b) c += self_couples(a, b);
+        return c;
     }
-    const T mr = S0.mut[v], mi = S0.kim;
-    T cr = T(1), ci = T(0);
-    for (int k = 0; k < kNMom; ++k) {
-        if (k > 0) {
-            const T nr = -(cr * mr - ci * mi) / T(k + 1);
-            const T ni = -(cr * mi + ci * mr) / T(k + 1);
-            cr = nr;
-            ci = ni;
-        }
-        if constexpr (sizeof(T) == 4) {
-            const T *__restrict__ M = A.momT + (size_t)k * K * K;
-            self_apply<K>(st0, cr, M, w0, std::make_integer_sequence<int, K>{});
-            self_apply<K>(st0, -ci, M, w1, std::make_integer_sequence<int, K>{});
-            self_apply<K>(st1, cr, M, w1, std::make_integer_sequence<int, K>{});
-            self_apply<K>(st1, ci, M, w0, std::make_integer_sequence<int, K>{});
-        } else {
-            const TA *__restrict__ M = A.mom + (size_t)k * K * K;
-#pragma unroll
-            for (int a = 0; a < K; ++a) {
-                T s0 = T(0), s1 = T(0);
-#pragma unroll
-                for (int b = 0; b < K; ++b) {
-                    s0 += T(M[a * K + b]) * w0[b];
-                    s1 += T(M[a * K + b]) * w1[b];
+    static constexpr int most()
+    {
+        int m = 0;
+        for (int a = 0; a < K; ++a) m = coupled(a) > m ? coupled(a) : m;
+        return m;
+    }
+    static constexpr int NJ = most();     // coupled coefficients of the self block
+    static constexpr int NZ = L / 2 + 1;  // z-power terms of a harmonic
+};
+
+// per coefficient: its coupled coefficients (ascending, padded with -1), and its
+// nonzero z-power terms (ascending, padded with -1)
+template <int L>
+struct CombTab {
+    using S = CombShape<L>;
+    short b[S::NJ][S::K], j[S::NZ][S::K];
+    double z[S::NZ][S::K];
+    constexpr CombTab() : b{}, j{}, z{}
+    {
+        for (int a = 0; a < S::K; ++a) {
+            for (int i = 0; i < S::NJ; ++i) b[i][a] = -1;
+            for (int i = 0; i < S::NZ; ++i) j[i][a] = -1;
+            int nb = 0, nz = 0;
+            for (int q = 0; q < S::K; ++q) {
+                if (self_couples(a, q)) b[nb++][a] = short(q);
+                if (kZPow<L>.m[a][q] != 0.0) {
+                    j[nz][a] = short(q);
+                    z[nz++][a] = kZPow<L>.m[a][q];
                 }
-                st0[a] += cr * s0 - ci * s1;
-                st1[a] += cr * s1 + ci * s0;
             }
         }
     }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const SolveDev<T, TA> &S = h ? S1 : S0;
-        TA acc[K];
-#pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] = TA(0);
-        for (int c = 0; c < A.nchunk; ++c) {
-            const T *__restrict__ p = S.part + ((size_t)c * g.N + v) * K;
-#pragma unroll
-            for (int a = 0; a < K; ++a) acc[a] += TA(p[a]);
+};
+template <int L>
+__constant__ constexpr CombTab<L> kCombTab{};
+
+template <typename T, typename TA, int L, int NH>
+__global__ __launch_bounds__(kCombThreads) void k_combine(CombArgs<T, TA> A, const SolveDev<T, TA> *__restrict__ sv)
+{
+    using Sh = CombShape<L>;
+    constexpr int K = Sh::K, VP = Sh::VP, VPT = Sh::VPT, VB = Sh::VB, NJ = Sh::NJ, NZ = Sh::NZ;
+    constexpr bool f32 = sizeof(T) == 4;
+    __shared__ TA zs[NH][VB * K];            // z-power sums, later A W
+    __shared__ TA bq[NH][VB * K];            // next term / n_a (stop rule); FP64: the self block before that
+    __shared__ T ws[NH][VB * K];             // W / n_a
+    __shared__ T cf[NH][kNMom][VB];          // series coefficients
+    __shared__ T ms[f32 ? kNMom * NJ * K : 1];  // packed moments [k][i][a]
+    const GridDev<T> &g = A.g;
+    const CombTab<L> &tab = kCombTab<L>;
+    const SolveDev<T, TA> *__restrict__ S = sv + NH * blockIdx.y;
+    const int tid = threadIdx.x, v0 = blockIdx.x * VB;
+    const bool live = tid < VP * K;
+    const int a = tid % K, q0 = tid / K;
+
+    if constexpr (f32) {
+        for (int q = tid; q < kNMom * NJ * K; q += kCombThreads) {
+            const int aa = q % K, i = (q / K) % NJ, k = q / (K * NJ), b = tab.b[i][aa];
+            ms[q] = b < 0 ? T(0) : A.momT[(size_t)k * K * K + aa * K + b];
         }
-        // the steps of k_combine, in its order
-        zpow_to_harmonic<TA, L>(acc);
+    }
+    if (tid < VB) {
+        const int v = min(v0 + tid, g.N - 1);
+        const T mr = S[0].mut[v];
+        T cr = T(1);
+        if constexpr (NH == 1) {
+            for (int k = 0; k < kNMom; ++k) {
+                if (k > 0) cr = cr * (-mr) / T(k + 1);
+                cf[0][k][tid] = cr;
+            }
+        } else {
+            const T mi = S[1].kim;
+            T ci = T(0);
+            for (int k = 0; k < kNMom; ++k) {
+                if (k > 0) {
+                    const T nr = -(cr * mr - ci * mi) / T(k + 1);
+                    const T ni = -(cr * mi + ci * mr) / T(k + 1);
+                    cr = nr;
+                    ci = ni;
+                }
+                cf[0][k][tid] = cr;
+                cf[1][k][tid] = ci;
+            }
+        }
+    }
+    const TA na = A.nsc[live ? a : 0];
+    TA acc[NH][VPT];
+    if (live) {
 #pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] *= A.nsc[a];
+        for (int h = 0; h < NH; ++h) {
+            const size_t e0 = (size_t)v0 * K + tid, cs = (size_t)g.N * K;
+            size_t e[VPT];
 #pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] += A.self_scale * TA(h ? st1[a] : st0[a]);
+            for (int i = 0; i < VPT; ++i) {
+                const bool in = v0 + i * VP + q0 < g.N;
+                e[i] = in ? e0 + (size_t)i * VP * K : a;  // beyond the grid: voxel 0's, not used
+                const T w = T(TA(S[h].W[e[i]]) / na);
+                ws[h][i * VP * K + tid] = in ? w : T(0);
+                acc[h][i] = TA(0);
+            }
+            const T *__restrict__ p = S[h].part;
+#pragma unroll 8
+            for (int c = 0; c < A.nchunk; ++c, p += cs) {
 #pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] *= A.dV;
-        combine_out<T, TA, L>(A, S, v, acc, h ? A.wsumI : A.wsum);
+                for (int i = 0; i < VPT; ++i) acc[h][i] += TA(p[e[i]]);
+            }
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) zs[h][i * VP * K + tid] = acc[h][i];
+        }
+    }
+    __syncthreads();
+    if constexpr (!f32) {
+        // self block on the matrix instruction: A = 16 rows of M_k (4 columns b at a
+        // time), B = W of 16 voxels; lane = (row or column n, column group gr)
+        typedef double d4 __attribute__((ext_vector_type(4)));
+        constexpr int RT = (K + 15) / 16, CT = (VB + 15) / 16, KS = (K + 3) / 4;
+        const int lane = tid & (kWave - 1), n = lane & 15, gr = lane >> 4;
+        for (int u = tid / kWave; u < RT * CT; u += kCombThreads / kWave) {
+            const int rt = u % RT, vv = (u / RT) * 16 + n, vc = min(vv, VB - 1), row = min(rt * 16 + n, K - 1);
+            double x[NH][KS], sum[NH][4];
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const int b = 4 * s + gr;
+                    const double w = ws[h][vc * K + min(b, K - 1)];
+                    x[h][s] = b < K ? w : 0.0;
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[h][r] = 0.0;
+            }
+            const gptr<double> M = as_global<double>(A.mom) + (size_t)row * K;
+            double mn[KS];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) mn[s] = M[min(4 * s + gr, K - 1)];
+#pragma unroll 1
+            for (int k = 0; k < kNMom; ++k) {
+                double m[KS];  // the next moment's entries are loaded under this one's products
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    m[s] = mn[s];
+                    mn[s] = M[(size_t)min(k + 1, kNMom - 1) * K * K + min(4 * s + gr, K - 1)];
+                }
+                d4 y[NH];
+#pragma unroll
+                for (int h = 0; h < NH; ++h) y[h] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+#pragma unroll
+                    for (int h = 0; h < NH; ++h)
+                        y[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[s], x[h][s], y[h], 0, 0, 0);
+                }
+                const double cr = cf[0][k][vc];
+                if constexpr (NH == 1) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[0][r] += cr * y[0][r];
+                } else {
+                    const double ci = cf[1][k][vc];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        sum[0][r] += cr * y[0][r] - ci * y[1][r];
+                        sum[1][r] += cr * y[1][r] + ci * y[0][r];
+                    }
+                }
+            }
+            // result r of a lane: row 4 r + gr, column n
+            if (vv < VB) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int ra = rt * 16 + 4 * r + gr;
+                    if (ra < K) {
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) bq[h][vv * K + ra] = sum[h][r];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const int P = g.nx * g.ny;
+    const bool edge = !A.op && (v0 < P || v0 + VB > g.N - P);  // the block holds voxels of the top or bottom face
+    if (live) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) acc[h][i] = TA(0);
+        }
+        // back to the harmonic basis
+#pragma unroll
+        for (int t = 0; t < NZ; ++t) {
+            const int j = tab.j[t][a];
+            const TA z = TA(tab.z[t][a]);
+            if (j >= 0) {
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                    for (int i = 0; i < VPT; ++i)
+                        acc[h][i] = fmad(z, zs[h][(i * VP + q0) * K + j], acc[h][i]);
+                }
+            }
+        }
+        TA st[NH][VPT];
+        if constexpr (f32) {
+            T w[NH][VPT][NJ], t32[NH][VPT];
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) {
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+                    t32[h][i] = T(0);
+#pragma unroll
+                    for (int t = 0; t < NJ; ++t) {
+                        const int b = tab.b[t][a];
+                        const T x = ws[h][(i * VP + q0) * K + (b < 0 ? a : b)];
+                        w[h][i][t] = b < 0 ? T(0) : x;
+                    }
+                }
+            }
+#pragma unroll 2
+            for (int k = 0; k < kNMom; ++k) {
+                T row[NH][VPT];
+#pragma unroll
+                for (int t = 0; t < NJ; ++t) {
+                    const T m = ms[(k * NJ + t) * K + a];
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                        for (int i = 0; i < VPT; ++i) row[h][i] = t ? fmad(m, w[h][i][t], row[h][i]) : m * w[h][i][t];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < VPT; ++i) {
+                    const T cr = cf[0][k][i * VP + q0];
+                    t32[0][i] = fmad(cr, row[0][i], t32[0][i]);
+                    if constexpr (NH == 2) {
+                        const T ci = cf[1][k][i * VP + q0];
+                        t32[0][i] = fmad(-ci, row[1][i], t32[0][i]);
+                        t32[1][i] = fmad(cr, row[1][i], t32[1][i]);
+                        t32[1][i] = fmad(ci, row[0][i], t32[1][i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                for (int i = 0; i < VPT; ++i) st[h][i] = TA(t32[h][i]);
+            }
+        } else {
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                for (int i = 0; i < VPT; ++i) st[h][i] = bq[h][i * VP * K + tid];
+            }
+        }
+        int l = 0;
+#pragma unroll
+        for (int ll = 1; ll <= L; ++ll) l += a >= ll * ll ? 1 : 0;
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            TA gl = TA(1);
+#pragma unroll
+            for (int ll = 1; ll <= L; ++ll) gl = ll <= l ? gl * TA(S[h].g) : gl;
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) {
+                const int v = v0 + i * VP + q0;
+                acc[h][i] = (acc[h][i] * na + A.self_scale * st[h][i]) * A.dV;
+                if (v >= g.N) continue;
+                const size_t e = (size_t)v * K + a;
+                if (A.op) {
+                    A.aw_out[e] = acc[h][i];
+                    continue;
+                }
+                if (S[h].aw_store) S[h].aw_store[e] = acc[h][i];
+                if (S[h].phi && S[h].mode != 3) S[h].phi[e] += acc[h][i];
+                if (S[h].mode == 0 || S[h].mode == 3) {
+                    const T wt = T(gl * TA(S[h].mus[v]) * acc[h][i] * na);
+                    S[h].W[e] = wt;
+                    if (edge) bq[h][i * VP * K + tid] = TA(wt) / na;
+                }
+            }
+        }
+    }
+    if (!edge) return;
+    __syncthreads();  // the z-power sums have been read
+    if (live) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) zs[h][i * VP * K + tid] = acc[h][i];
+        }
+    }
+    __syncthreads();
+    // the faces' functionals: one thread per voxel and half
+    for (int t = tid; t < NH * VB; t += kCombThreads) {
+        const int h = t / VB, q = t - h * VB, v = v0 + q;
+        const SolveDev<T, TA> &X = S[h];
+        if (v >= g.N || X.mode == 3) continue;
+        const TA *f = &zs[h][q * K];
+        if (v >= g.N - P) {
+            const int pix = v - (g.N - P);
+            TA e = TA(0);
+#pragma unroll
+            for (int l = 0; l <= L; ++l) e += A.coefE[l] * f[l * l + l];
+            X.dE[pix] = e;
+            if (X.mode == 0) {
+                TA bs = TA(0);
+                for (int c = 0; c < K; ++c) bs += (h ? A.wsumI : A.wsum)[c] * bq[h][q * K + c];
+                X.bsum[pix] = bs;
+            }
+        }
+        if (v < P) {
+            TA r = TA(0);
+#pragma unroll
+            for (int l = 0; l <= L; ++l) r += A.coefR[l] * f[l * l + l];
+            X.dR[v] = r;
+        }
     }
 }
 
@@ -1157,8 +1312,11 @@ template <typename T, typename TA>
 hipError_t launch_combine(int L, const CombArgs<T, TA> &A, const SolveDev<T, TA> *sv, int nsolve,
                           hipStream_t st)
 {
-    dim3 grid((A.g.N + kWave - 1) / kWave, nsolve), block(kWave);
-    RTE_DISPATCH_L(L, hipLaunchKernelGGL((k_combine<T, TA, LL>), grid, block, 0, st, A, sv));
+    RTE_DISPATCH_L(L, {
+        constexpr int VB = CombShape<LL>::VB;
+        hipLaunchKernelGGL((k_combine<T, TA, LL, 1>), dim3((A.g.N + VB - 1) / VB, nsolve), dim3(kCombThreads), 0, st,
+                           A, sv);
+    });
     return hipGetLastError();
 }
 
@@ -1166,8 +1324,11 @@ template <typename T, typename TA>
 hipError_t launch_combine_c(int L, const CombArgs<T, TA> &A, const SolveDev<T, TA> *sv, int ncomplex,
                             hipStream_t st)
 {
-    dim3 grid((A.g.N + kWave - 1) / kWave, ncomplex), block(kWave);
-    RTE_DISPATCH_L(L, hipLaunchKernelGGL((k_combine_c<T, TA, LL>), grid, block, 0, st, A, sv));
+    RTE_DISPATCH_L(L, {
+        constexpr int VB = CombShape<LL>::VB;
+        hipLaunchKernelGGL((k_combine<T, TA, LL, 2>), dim3((A.g.N + VB - 1) / VB, ncomplex), dim3(kCombThreads), 0,
+                           st, A, sv);
+    });
     return hipGetLastError();
 }
 

@@ -31,6 +31,13 @@ template <>
 __host__ __device__ __forceinline__ double fmad<double>(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 template <typename T>
+__device__ __forceinline__ T dev_min(T a, T b);
+template <>
+__device__ __forceinline__ float dev_min<float>(float a, float b) { return __builtin_fminf(a, b); }
+template <>
+__device__ __forceinline__ double dev_min<double>(double a, double b) { return __builtin_fmin(a, b); }
+
+template <typename T>
 __device__ __forceinline__ T dev_exp(T x);
 template <>
 __device__ __forceinline__ float dev_exp<float>(float x) { return expf(x); }

@@ -345,104 +345,158 @@ __global__ __launch_bounds__(256) void k_to_zpow(int N, const SolveDev<T, TA> *_
 // ---------------------------------------------------------------------------
 // Per-medium table kf(d, s) = e^{-tau(d,s)}/r^2 (0 for d == s, r >= thresh and
 // padding), layout [s][slot(d)].  The ray between two voxel centres is the
-// same both ways, so one wave marches the pairs of a brick pair (bd, bs) with
-// bs <= bd once (from s to d) and writes both entries: the direct one
-// (row s, the wave's 64 destination slots: one coalesced row segment per
-// source) and, off the diagonal, the mirrored one (row d, the source brick's
-// slots), held in registers and written as one 256-byte run per lane after the
-// brick's march (FP32; FP64 one x row of 4 sources at a time).  mu_t is read
-// from LDS when the whole map fits.
-// grid = ceil(ntiles / waves per block), block = KT threads.
+// same both ways, so a pair of bricks (bs, bd = bs + D) is marched once (from s to
+// d), D in the half space z, then y, then x >= 0, and both entries are written: the
+// direct one (row s, the brick's 64 destination slots: one coalesced row segment
+// per source) and, off the diagonal, the mirrored one (row d, the source brick's
+// slots): a lane's SG mirrored entries stay in registers and go out as one run
+// (16 of FP32 are 64 bytes; 16-byte pieces reached HBM as partly filled lines,
+// 2.1x the table's bytes).
+// A ray's crossings depend on its displacement alone, and every translation of a
+// brick pair has the same 64 x 64 displacements: a wave (lane = destination of the
+// brick) marches M translated pairs together, one sequence of crossings and
+// per pair and crossing one address, one read of mu_t and one FMA.  (Marched pair by
+// pair a crossing cost ~17 vector instructions, which bounded the table; now it is
+// 13 / M + 2.)  Measured, before -> now: FP32 8^3 0.157 -> 0.020 ms, 16^3 0.29 -> 0.079,
+// 24^3 1.98 -> 0.51, 32^3 12.0 -> 3.2 (1.3 TB/s written; vector issue), 34^3 23 -> 8.7;
+// FP64 24^3 3.07 -> 1.0.
+// MEM 0: mu_t from memory; 1: from LDS, the map followed by what the padded voxels
+// of the last bricks reach; 2: from LDS without that tail.  0 and 2 clamp the
+// index of each read (a padded voxel's path; its entry is 0 whatever is read).
+// grid = at most the resident blocks; unit u (translation group, D, SG of the source
+// brick's 64 voxels) belongs to block u mod grid, whose waves share its units.
 // ---------------------------------------------------------------------------
-template <typename T, bool LDS>
-__global__ __launch_bounds__(1024) void k_ktab(GridDev<T> g, int ntiles, T thr2, const T *__restrict__ mut,
-                                               T *__restrict__ ktab)
+// r^2 with its roundings fixed: a pair at exactly the threshold radius stays on its side
+template <typename T>
+__device__ __forceinline__ T sum_squares(T x, T y, T z)
+{
+#pragma clang fp contract(off)
+    return fmad(x, x, y * y) + z * z;
+}
+
+struct KtabPlan {
+    int py, pz;       // pitches of y and z in the map read (elements)
+    int last;         // largest index of the map read
+    int nD, nunits;
+    int next;         // where in LDS the block's unit counter lies (bytes), -1: no room
+};
+
+template <typename T, int MEM, int M, int SG, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T thr2, const T *__restrict__ mut,
+                                                  T *__restrict__ ktab)
 {
     extern __shared__ __align__(16) unsigned char ktab_lds[];
+    constexpr int NS = kWave / SG;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    if constexpr (LDS) {
-        T *sm = reinterpret_cast<T *>(ktab_lds);
-        for (int i = tid; i < g.N; i += blockDim.x) sm[i] = mut[i];
-        __syncthreads();
-    }
-    const int tile = blockIdx.x * (blockDim.x / kWave) + tid / kWave;
-    if (tile >= ntiles) return;
-    // tile -> (bd, bs), bs <= bd
-    int bd = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
-    while (bd > 0 && bd * (bd + 1) / 2 > tile) --bd;
-    while ((bd + 1) * (bd + 2) / 2 <= tile) ++bd;
-    const int bs = tile - bd * (bd + 1) / 2;
-    int di, dj, dk;
-    lane_dest(g, bd, lane, di, dj, dk);
-    const bool dvalid = di < g.nx && dj < g.ny && dk < g.nz;
-    const int cdi = min(di, g.nx - 1), cdj = min(dj, g.ny - 1), cdk = min(dk, g.nz - 1);
     const int nxy = g.nx * g.ny;
-    const int dslot = bd * kWave + lane;
-    const int dlin = cdi + g.nx * cdj + nxy * cdk;
-    const int bxi = bs % g.bx, byi = (bs / g.bx) % g.by, bzi = bs / (g.bx * g.by);
-    const bool mirror = bs != bd;
-    // kf of source (si, sj, sk) of the brick for this lane's destination, written
-    // to the direct entry (row s, this wave's 64 slots: one coalesced segment)
-    auto entry = [&](int jj, int q) -> T {
-        const int si = bxi * kBrick + jj, sj = byi * kBrick + (q & 3), sk = bzi * kBrick + (q >> 2);
-        T kf = T(0);
-        if (si < g.nx && sj < g.ny && sk < g.nz) {  // wave-uniform
-            const int ix = cdi - si, iy = cdj - sj, iz = cdk - sk;
-            const T ddx = T(ix) * g.dx, ddy = T(iy) * g.dy, ddz = T(iz) * g.dz;
-            const T r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-            const bool self = (ix == 0) && (iy == 0) && (iz == 0);
-            const bool use = dvalid && !self && (r2 < thr2);
-            const T r = sqrt(self ? T(1) : r2);
-            const int slin = si + g.nx * sj + nxy * sk;
-            T tau = T(0);
-            if (use) {
-                if constexpr (LDS)
-                    tau = march_tau<T>((const __attribute__((address_space(3))) T *)ktab_lds, slin, ix, iy, iz, g.nx,
-                                       nxy, r);
-                else
-                    tau = march_tau<T>(as_global<T>(mut), slin, ix, iy, iz, g.nx, nxy, r);
-            }
-            kf = use ? dev_exp<T>(-tau) / r2 : T(0);
-            ktab[(size_t)slin * g.npad + dslot] = kf;
+    if constexpr (MEM != 0) {
+        T *sm = reinterpret_cast<T *>(ktab_lds);
+        for (int i = tid; i < g.N; i += THREADS) {
+            const int x = i % g.nx, y = (i / g.nx) % g.ny, z = i / nxy;
+            sm[x + p.py * y + p.pz * z] = mut[i];
         }
-        return kf;
+    }
+    int *next = reinterpret_cast<int *>(ktab_lds + p.next);
+    if (p.next >= 0 && tid == 0) *next = 0;
+    __syncthreads();
+    const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+    const int ex = 2 * g.bx - 1, ey = 2 * g.by - 1;
+    auto mu_at = [&](int i) -> T {
+        if constexpr (MEM != 1) i = min(i, p.last);
+        if constexpr (MEM != 0)
+            return ((const __attribute__((address_space(3))) T *)ktab_lds)[i];
+        else
+            return as_global<T>(mut)[i];
     };
-    using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-    constexpr int per = sizeof(V) / sizeof(T);
-    V *row = reinterpret_cast<V *>(ktab + (size_t)dlin * g.npad + bs * kWave);
-    if constexpr (sizeof(T) == 4) {
-        // FP32: the brick's 64 mirrored entries stay in registers and go out as one
-        // 256-byte run per lane after the march (written piecewise, the rows' lines
-        // reached HBM partly filled: 2.1x the table's bytes)
-        T m[kWave];
+    for (int own = tid / kWave;; own += THREADS / kWave) {
+        // the block's next unit (in a fixed order where its map leaves no room for a counter)
+        if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
+        const int u = blockIdx.x + gridDim.x * __builtin_amdgcn_readfirstlane(own);
+        if (u >= p.nunits) break;
+        const int slab = u % NS, f = (u / NS) % p.nD + p.nD - 1, first = (u / NS) / p.nD * M;
+        const int Dx = f % ex - (g.bx - 1), Dy = (f / ex) % ey - (g.by - 1), Dz = f / (ex * ey) - (g.bz - 1);
+        const int cx = g.bx - abs(Dx), cy = g.by - abs(Dy), cnt = cx * cy * (g.bz - abs(Dz));
+        if (first >= cnt) continue;
+        const bool mirror = (Dx | Dy | Dz) != 0;
+        // the M source bricks (the last one again where there are fewer): voxel (0,0,0) of each
+        int bx0[M], by0[M], bz0[M];
 #pragma unroll
-        for (int q = 0; q < 16; ++q)  // the source brick's x rows, 4 voxels each
+        for (int m = 0; m < M; ++m) {
+            const int t = min(first + m, cnt - 1);
+            bx0[m] = (t % cx + max(0, -Dx)) * kBrick;
+            by0[m] = ((t / cx) % cy + max(0, -Dy)) * kBrick;
+            bz0[m] = (t / (cx * cy) + max(0, -Dz)) * kBrick;
+        }
+        T mir[M][SG];
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) m[q * 4 + jj] = entry(jj, q);
-        if (mirror && dvalid) {
+        for (int i = 0; i < SG; ++i) {
+            const int j = slab * SG + i, sx = j & 3, sy = (j >> 2) & 3, sz = j >> 4;
+            const int ix = Dx * kBrick + lx - sx, iy = Dy * kBrick + ly - sy, iz = Dz * kBrick + lz - sz;
+            const T ddx = T(ix) * g.dx, ddy = T(iy) * g.dy, ddz = T(iz) * g.dz;
+            const T r2 = sum_squares(ddx, ddy, ddz);
+            const bool self = (ix == 0) && (iy == 0) && (iz == 0);
+            const bool use = !self && r2 < thr2;
+            const T r = sqrt(self ? T(1) : r2);
+            // march_tau for M starting voxels
+            const int n0 = abs(ix), n1 = abs(iy), n2 = abs(iz);
+            const T BIG = big_value<T>();
+            const T inc0 = n0 ? T(1) / T(n0) : BIG, inc1 = n1 ? T(1) / T(n1) : BIG, inc2 = n2 ? T(1) / T(n2) : BIG;
+            T a0 = T(0.5) * inc0, a1 = T(0.5) * inc1, a2 = T(0.5) * inc2;
+            const int st0 = ix > 0 ? 1 : -1, st1 = iy > 0 ? p.py : -p.py, st2 = iz > 0 ? p.pz : -p.pz;
+            const int nsteps = use ? n0 + n1 + n2 : 0;
+            int s0[M], v = 0;
+            T mu[M], acc[M], prev = T(0);
 #pragma unroll
-            for (int u = 0; u < kWave / per; ++u) {
-                V x;
-                T *xs = reinterpret_cast<T *>(&x);
+            for (int m = 0; m < M; ++m) {
+                s0[m] = bx0[m] + sx + p.py * (by0[m] + sy) + p.pz * (bz0[m] + sz);
+                mu[m] = mu_at(s0[m]);
+                acc[m] = T(0);
+            }
+            for (int t = 0; t < nsteps; ++t) {
+                const T a = dev_min(dev_min(a0, a1), a2);
+                const bool pz = a2 == a, py = !pz && a1 == a;
+                v += pz ? st2 : (py ? st1 : st0);
+                const T len = a - prev;
+                prev = a;
 #pragma unroll
-                for (int e = 0; e < per; ++e) xs[e] = m[u * per + e];
-                row[u] = x;
+                for (int m = 0; m < M; ++m) {
+                    acc[m] += mu[m] * len;
+                    mu[m] = mu_at(v + s0[m]);
+                }
+                a2 = pz ? a2 + inc2 : a2;
+                a1 = py ? a1 + inc1 : a1;
+                a0 = (!pz && !py) ? a0 + inc0 : a0;
+            }
+            const T last = T(0.5) * dev_min(dev_min(inc0, inc1), inc2);
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int x = bx0[m] + sx, y = by0[m] + sy, z = bz0[m] + sz;
+                const bool sv = x < g.nx && y < g.ny && z < g.nz;
+                const bool dv = x + ix < g.nx && y + iy < g.ny && z + iz < g.nz;
+                const T tau = (acc[m] + mu[m] * last) * r;
+                const T kf = use && dv && sv ? dev_exp<T>(-tau) / r2 : T(0);
+                mir[m][i] = kf;
+                const int bd = (bx0[m] / kBrick + Dx) + g.bx * ((by0[m] / kBrick + Dy) + g.by * (bz0[m] / kBrick + Dz));
+                if (sv && first + m < cnt)
+                    ktab[(size_t)(x + g.nx * y + nxy * z) * g.npad + bd * kWave + lane] = kf;
             }
         }
-    } else {
-        // FP64: one x row of 4 sources at a time (the whole brick would spill)
-        for (int q = 0; q < 16; ++q) {
-            T m[4];
+        if (!mirror) continue;
+        using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
+        constexpr int per = sizeof(V) / sizeof(T);
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) m[jj] = entry(jj, q);
-            if (mirror && dvalid) {
+        for (int m = 0; m < M; ++m) {
+            const int x = bx0[m] + Dx * kBrick + lx, y = by0[m] + Dy * kBrick + ly, z = bz0[m] + Dz * kBrick + lz;
+            const int bs = bx0[m] / kBrick + g.bx * (by0[m] / kBrick + g.by * (bz0[m] / kBrick));
+            if (first + m < cnt && x < g.nx && y < g.ny && z < g.nz) {
+                V *row = reinterpret_cast<V *>(ktab + (size_t)(x + g.nx * y + nxy * z) * g.npad + bs * kWave + slab * SG);
 #pragma unroll
-                for (int u = 0; u < 4 / per; ++u) {
-                    V x;
-                    T *xs = reinterpret_cast<T *>(&x);
+                for (int w = 0; w < SG / per; ++w) {
+                    V o;
+                    T *os = reinterpret_cast<T *>(&o);
 #pragma unroll
-                    for (int e = 0; e < per; ++e) xs[e] = m[u * per + e];
-                    row[q * 4 / per + u] = x;
+                    for (int e = 0; e < per; ++e) os[e] = mir[m][w * per + e];
+                    row[w] = o;
                 }
             }
         }
@@ -1278,34 +1332,70 @@ hipError_t launch_prop_c(int L, int path, const PropArgs<T> &A, const SolveDev<T
     return hipGetLastError();
 }
 
+template <typename T, int MEM, int M, int SG, int THREADS>
+static hipError_t launch_ktab_as(const GridDev<T> &g, KtabPlan p, size_t lds, int cus, T thr2, const T *mut, T *ktab,
+                                 hipStream_t st)
+{
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ktab<T, MEM, M, SG, THREADS>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    constexpr int waves = THREADS / kWave;
+    p.nunits = p.nD * ((g.nblk + M - 1) / M) * (kWave / SG);
+    const int blocks = min((p.nunits + waves - 1) / waves, cus * (1024 / THREADS));
+    hipLaunchKernelGGL((k_ktab<T, MEM, M, SG, THREADS>), dim3(blocks), dim3(THREADS), lds, st, g, p, thr2, mut, ktab);
+    return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_ktab(const GridDev<T> &g, T thr2, const T *mut, T *ktab, hipStream_t st)
 {
-    static int lds_max = -1;
+    static int lds_max = -1, cus = 0;
     if (lds_max < 0) {
         int dev = 0, v = 0;
         hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
         if (e != hipSuccess) return e;
         lds_max = v;
     }
-    const int ntiles = g.nblk * (g.nblk + 1) / 2;
-    const size_t lds = (size_t)g.N * sizeof(T);
-    if (lds <= (size_t)lds_max) {
-        constexpr int threads = 1024;
-        if (lds > 65536) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ktab<T, true>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        const int blocks = (ntiles + threads / kWave - 1) / (threads / kWave);
-        hipLaunchKernelGGL((k_ktab<T, true>), dim3(blocks), dim3(threads), lds, st, g, ntiles, thr2, mut, ktab);
-    } else {
-        constexpr int threads = 256;
-        const int blocks = (ntiles + threads / kWave - 1) / (threads / kWave);
-        hipLaunchKernelGGL((k_ktab<T, false>), dim3(blocks), dim3(threads), 0, st, g, ntiles, thr2, mut, ktab);
+    // LDS pitches: y = 4 (mod 8), z = 16 (mod 32) put the 64 voxels of a brick in
+    // different banks (5 % at 24^3 and 32^3); the plain map where that does not fit
+    KtabPlan p{};
+    size_t map = 0, lds = 0;
+    auto fits = [&](bool tail) {
+        p.last = tail ? 4 * g.bx - 1 + p.py * (4 * g.by - 1) + p.pz * (4 * g.bz - 1)
+                      : g.nx - 1 + p.py * (g.ny - 1) + p.pz * (g.nz - 1);
+        map = ((size_t)(p.last + 1) * sizeof(T) + 15) / 16 * 16;
+        p.next = map + 16 <= (size_t)lds_max ? (int)map : -1;
+        lds = p.next >= 0 ? map + 16 : map;
+        return lds <= (size_t)lds_max;
+    };
+    p.py = g.nx + (12 - g.nx % 8) % 8;
+    p.pz = p.py * g.ny + (48 - p.py * g.ny % 32) % 32;
+    int mem = 1;
+    if (!fits(true)) {
+        p.py = g.nx;
+        p.pz = g.nx * g.ny;
+        if (!fits(true)) mem = fits(false) ? 2 : 0;
     }
-    return hipGetLastError();
+    if (mem == 0) {
+        p.next = 0;
+        lds = 16;
+    }
+    p.nD = ((2 * g.bx - 1) * (2 * g.by - 1) * (2 * g.bz - 1) + 1) / 2;
+    // 7 translations and 8 sources per unit (FP64: 8 and 4, at half the waves) -- the most
+    // that 1024 threads hold without scratch -- while that leaves the chip's waves several
+    // units, else 4 and 4 (more, shorter units).  Either way in ms: 12^3 0.036 / 0.028,
+    // 16^3 0.079 / 0.078, 18^3 0.197 / 0.264, 20^3 0.192 / 0.266, 32^3 3.2 / 3.7
+    const bool wide = (long long)g.nblk * (g.nblk + 1) / 2 >= 16LL * cus;
+    constexpr bool f32 = sizeof(T) == 4;
+#define RTE_KTAB(MEM)                                                                                           \
+    (wide ? launch_ktab_as<T, MEM, f32 ? 7 : 8, f32 ? 8 : 4, f32 ? 1024 : 512>(g, p, lds, cus, thr2, mut, ktab, st) \
+          : launch_ktab_as<T, MEM, 4, 4, 256>(g, p, lds, cus, thr2, mut, ktab, st))
+    return mem == 1 ? RTE_KTAB(1) : mem == 2 ? RTE_KTAB(2) : RTE_KTAB(0);
+#undef RTE_KTAB
 }
 
 template <typename T, typename TA>

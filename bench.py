@@ -26,6 +26,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3   # MI355X FP32 (vector/matrix dense) published peak
+PEAK_F16_MFMA_TFLOPS = 2500.0  # MI355X FP16 matrix, dense
 PEAK_HBM_GBS = 8000.0
 # HBM bytes per solve and term of k_prop at 32^3 L=5 (mixed, cached), from rocprofv3
 # FETCH_SIZE + WRITE_SIZE calibrated against a device copy: a beam in a group of five,
@@ -596,9 +597,11 @@ def main():
     value = nsolve / (ms_per_step / 1000.0)
     terms_mean = float(np.mean([s["terms"] for s in stats]))
 
-    # roofline of the dominant kernel, the propagation group of the default size
-    # (k_prop<float, double, L, 0, 5>; the library allows at most 3 at L = 6 and 2 from
-    # L = 7): its algorithmic flops / its launch time
+    # roofline of the dominant kernel: k_prop_mfma on the grids and orders that the library
+    # runs on the matrix cores (groups of five and more beams counted under 5), else the
+    # propagation group of the default size (k_prop<float, double, L, 0, 5>; the library
+    # allows at most 3 at L = 6 and 2 from L = 7): its algorithmic flops / its launch time
+    on_mfma = L in (4, 5) and n >= 32
     gsz = min(args.group or DEFAULT_GROUP, args.beams, 5 if L <= 5 else (3 if L == 6 else 2))
     launches = max(prof["group_launches"][gsz], 1)
     avg_ms = prof["group_ms"][gsz] / launches
@@ -611,8 +614,12 @@ def main():
     npairs = float(n ** 3) * (n ** 3 - 1)
     # beam-terms a launch processes: the library counts (16 + k 4K) flops per pair of a group of k
     beam_terms = flops_per_launch / ((16 + gsz * 4 * K) * npairs) * gsz
+    # the matrix flops that k_prop_mfma executes: FP16 products of two pieces each, 10 (L = 4: 7)
+    # of 16 x 16 x 32 per 16 sources x 16 destinations x 16 columns and source (or destination)
+    executed = achieved * (10 if L == 5 else 7) * 64.0 / (4 * K)
+    peak = PEAK_F16_MFMA_TFLOPS if on_mfma else PEAK_FP32_TFLOPS
     traffic = None
-    if n == 32 and L == 5 and gsz in TRAFFIC_PER_SOLVE_TERM:
+    if n == 32 and L == 5 and gsz in TRAFFIC_PER_SOLVE_TERM and not on_mfma:
         traffic = TRAFFIC_PER_SOLVE_TERM[gsz] * beam_terms
 
     out = {}
@@ -670,9 +677,12 @@ def main():
                                % nsolve},
         "terms_mean": terms_mean,
         "voxel_pair_propagations_per_s": pairs_per_s,
-        "roofline": {"bound": "valu", "pipe": "valu-fp32", "achieved": achieved, "peak": PEAK_FP32_TFLOPS,
-                     "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic,
-                     "kernel": "k_prop<float, double, %d, 0, %d> (groups of %d beams, cached path)" % (L, gsz, gsz),
+        "roofline": {"bound": "mfma" if on_mfma else "valu", "pipe": "mfma-f16" if on_mfma else "valu-fp32",
+                     "achieved": executed if on_mfma else achieved, "peak": peak,
+                     "unit": "TFLOP/s", "frac": (executed if on_mfma else achieved) / peak, "traffic": traffic,
+                     "algorithmic_tflops": achieved,
+                     "kernel": "k_prop_mfma<double, %d> (groups of five and more solves, cached path)" % L if on_mfma else
+                               "k_prop<float, double, %d, 0, %d> (groups of %d beams, cached path)" % (L, gsz, gsz),
                      "launches": launches, "avg_launch_ms": avg_ms, "flops_per_launch": flops_per_launch,
                      "beam_terms_per_launch": beam_terms,
                      "all_propagation_launches": {"launches": all_launches,

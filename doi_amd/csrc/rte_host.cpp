@@ -16,6 +16,8 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
+#include <list>
+#include <mutex>
 #include <map>
 #include <memory>
 #include <set>
@@ -296,6 +298,12 @@ struct MomentSet {
     DevBuf md, mf;  // [kNMom][K][K] in double and float
 };
 
+// Z pieces of a grid's displacements (rte_mfma.hip), shared with the calls and buckets using it
+struct ZTab {
+    std::tuple<int, int, int, int, double, double, double> key;  // L, brick counts, nz, spacings
+    std::shared_ptr<DevBuf> buf;
+};
+
 struct PendingTiming {
     int kind;  // 0 prop, 1 ktab, 2 other
     hipEvent_t a, b;
@@ -313,6 +321,8 @@ struct rte_ctx {
     std::vector<hipEvent_t> ev_pool;
     std::vector<PendingTiming> pending;
     std::map<std::tuple<int, double, double, double>, std::unique_ptr<MomentSet>> moments;
+    std::list<ZTab> ztabs;  // Z tables of the matrix-core propagation, last used first
+    std::mutex ztabs_mu;    // (a server's thread uses them too)
     // solve workspace (grow-only)
     DevBuf ws_W, ws_Wp, ws_part, ws_pix, ws_sv, ws_beams, ws_red;
     std::set<rte_medium *> media;  // live media of this context
@@ -330,6 +340,8 @@ struct rte_medium {
     DevBuf mut_d;                 // FP64 mu_t
     DevBuf ktab_f, ktab_d;        // cached e^{-tau}/r^2 tables
     double ktab_f_thr = -1, ktab_d_thr = -1;
+    DevBuf kexp;  // exponents of ktab_f, if kexp_ok
+    bool kexp_ok = false;
 };
 
 static int set_device(rte_ctx *ctx)
@@ -597,6 +609,8 @@ extern "C" int rte_medium_reset_cache(rte_medium *m)
     m->ktab_f.release();
     m->ktab_d.release();
     m->ktab_f_thr = m->ktab_d_thr = -1;
+    m->kexp.release();
+    m->kexp_ok = false;
     return RTE_OK;
 }
 
@@ -660,6 +674,7 @@ static int ensure_ktab(rte_medium *m, double thr, hipStream_t on = nullptr)
     double &tthr = sizeof(T) == 4 ? m->ktab_f_thr : m->ktab_d_thr;
     if (tab.p && tthr == thr) return RTE_OK;
     const GridDev<T> g = make_grid<T>(m->grid);
+    if (sizeof(T) == 4) m->kexp_ok = false;
     HIP_TRY(tab.alloc((size_t)g.N * g.npad * sizeof(T)));
     const T *mut = sizeof(T) == 4 ? (const T *)m->mut_f.p : (const T *)m->mut_d.p;
     const T thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
@@ -672,6 +687,151 @@ static int ensure_ktab(rte_medium *m, double thr, hipStream_t on = nullptr)
     }
     tthr = thr;
     return RTE_OK;
+}
+
+// the exponents of a medium's FP32 path table, for the matrix-core propagation
+static int ensure_kexp(rte_medium *m)
+{
+    if (m->kexp_ok) return RTE_OK;
+    const GridDev<float> g = make_grid<float>(m->grid);
+    HIP_TRY(m->kexp.alloc(kexp_bytes(g)));
+    LaunchTimer tm(m->ctx, 1);
+    HIP_TRY(launch_kexp(g, m->ktab_f.as<float>(), m->kexp.as<unsigned char>(), m->ctx->stream));
+    tm.done();
+    m->kexp_ok = true;
+    return RTE_OK;
+}
+
+// ---- how a grid's propagation runs ------------------------------------------
+// Chunks (of source brick rows) of the matrix-core propagation of a solve alone, and its
+// estimated time in us: rounds of its workgroups over 256 CUs, each one's tiles (a source
+// slab, 4.3 us) and its start, and the partial sums' way through memory.
+static double mfma_chunks(const GridDev<float> &g, int K, int *nchunk)
+{
+    int tx = 1, tz = 1;
+    const double tiles = mfma_translations(g, 1, &tx, &tz);
+    const double units = (double)((g.bx + tx - 1) / tx) * g.by * ((g.bz + tz - 1) / tz);
+    double best = 0;
+    *nchunk = 1;
+    for (int y = 1; y <= g.by; ++y) {
+        const double rounds = std::ceil(units * y / 256.0);
+        const double each = tiles / units / g.by * ((g.by + y - 1) / y) + 4.0;
+        const double cost = rounds * each * 4.3 + (double)y * g.N * K * 8.0 / 3e6;
+        if (best == 0 || cost < best) {
+            best = cost;
+            *nchunk = y;
+        }
+    }
+    return best;
+}
+
+// Whether the FP32 cached propagation of a grid runs on the matrix cores (rte_mfma.hip):
+// L = 4 and 5, where a solve alone is to take at most 0.95 of k_prop's time there (2.34
+// and 2.94 ps a pair), which is where no group of solves measured slower.  It depends on
+// the grid and order only, so that a solve takes the same kernel, and has the same bits,
+// alone and in any batch.
+static bool use_mfma(int L, const GridDev<float> &g)
+{
+    if (L != 4 && L != 5) return false;
+    int nch = 1;
+    return mfma_chunks(g, (L + 1) * (L + 1), &nch) < 0.95 * (L == 4 ? 2.34e-6 : 2.94e-6) * g.N * (double)g.N;
+}
+
+// The chunks of a propagation and the size of its input copy Wp (in T); depends on
+// the grid, order and path only, so that a solve's partial sums, and its bits, are the
+// same alone and in any batch.
+struct PropShape {
+    bool mfma = false;
+    int nch = 1, clen = 0;
+    size_t wp = 0;
+};
+
+template <typename T>
+static PropShape prop_shape(const GridDev<T> &g, int L, int path, bool cplx)
+{
+    PropShape s;
+    const int K = (L + 1) * (L + 1);
+    if constexpr (sizeof(T) == 4) {
+        if (path == RTE_PATH_CACHED && !cplx && use_mfma(L, g)) {
+            s.mfma = true;
+            mfma_chunks(g, K, &s.nch);
+            s.wp = mfma_wp_bytes(L, g) / sizeof(T);
+            return s;
+        }
+    }
+    const int nch0 = pick_chunks(g.nblk, 1, g.N);
+    s.clen = (g.N + nch0 - 1) / nch0;
+    s.nch = (g.N + s.clen - 1) / s.clen;
+    s.wp = (size_t)g.N * K;
+    return s;
+}
+
+// The Z table of a grid and order, built on first use; the least recently used ones
+// beyond kZTabKeep bytes are dropped (freed when their last user lets go).
+constexpr size_t kZTabKeep = size_t(1) << 30;
+static int get_ztab(rte_ctx *ctx, int L, const GridDev<float> &g, double dx, double dy, double dz, hipStream_t st,
+                    std::shared_ptr<DevBuf> *out)
+{
+    const auto key = std::make_tuple(L, g.bx, g.by, g.nz, dx, dy, dz);
+    std::lock_guard<std::mutex> lk(ctx->ztabs_mu);
+    for (auto it = ctx->ztabs.begin(); it != ctx->ztabs.end(); ++it)
+        if (it->key == key) {
+            ctx->ztabs.splice(ctx->ztabs.begin(), ctx->ztabs, it);
+            *out = it->buf;
+            return RTE_OK;
+        }
+    auto buf = std::make_shared<DevBuf>();
+    HIP_TRY(buf->alloc(mfma_ztab_bytes(L, g)));
+    HIP_TRY(launch_ztab(L, g, dx, dy, dz, buf->as<unsigned char>(), st));
+    HIP_TRY(hipStreamSynchronize(st));  // other streams may use it next
+    ctx->ztabs.push_front(ZTab{key, buf});
+    size_t kept = 0;
+    for (auto it = ctx->ztabs.begin(); it != ctx->ztabs.end();) {
+        kept += it->buf->bytes;
+        it = kept > kZTabKeep && it != ctx->ztabs.begin() ? ctx->ztabs.erase(it) : std::next(it);
+    }
+    *out = buf;
+    return RTE_OK;
+}
+
+// The launch arguments of a propagation; zt keeps the Z table alive for the caller.
+template <typename T>
+static int prop_args(rte_ctx *ctx, const GridDev<T> &g, const rte_grid &grid, int L, const PropShape &sh, double thr,
+                     hipStream_t st, PropArgs<T> *pa, std::shared_ptr<DevBuf> *zt)
+{
+    pa->g = g;
+    pa->nchunk = sh.nch;
+    pa->chunk_len = sh.clen;
+    pa->thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
+    if constexpr (sizeof(T) == 4) {
+        if (sh.mfma) {
+            const int rc = get_ztab(ctx, L, g, (grid.xmax - grid.xmin) / grid.nx, (grid.ymax - grid.ymin) / grid.ny,
+                                    (grid.zmax - grid.zmin) / grid.nz, st, zt);
+            if (rc) return rc;
+            pa->zt = (*zt)->template as<unsigned char>();
+        }
+    }
+    return RTE_OK;
+}
+
+// Sizes of the groups that n solves on the matrix cores go in: a group's columns are its
+// solves times as many translations as fit in 16; a translation costs the bricks at which
+// not every column has a source, an unused column its share of every product.  Whole
+// groups of 16, 15 as one, and what is left in powers of two (thousand tiles per solve
+// and term at 32^3: 66 in a group of 16, 74 of 8, 83 of 4, 101 of 2, 124 alone).
+static std::vector<int> mfma_groups(int n, int most)
+{
+    std::vector<int> out;
+    for (int k = most; n > 0;) {
+        if (n >= k || (most == kMfmaCols && n == kMfmaCols - 1)) {
+            out.push_back(std::min(n, k));
+            n -= out.back();
+        } else {
+            k = 1;
+            while (2 * k <= n) k *= 2;
+        }
+    }
+    return out;
 }
 
 // ---------------------------------------------------------------------------
@@ -812,14 +972,17 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
         for (int i = 0; i < nb; ++i)
             if ((rc = ensure_ktab<T>(media[i], thr))) return rc;
 
-    // the source chunking depends on the grid only, so a solve's partial sums,
-    // and so its result bits, are the same alone and in any batch
-    const int nchunk = pick_chunks(g.nblk, 1, N);
-    const int clen = (N + nchunk - 1) / nchunk;
-    const int nch = (N + clen - 1) / clen;
+    const PropShape sh = prop_shape<T>(g, L, path, kim != nullptr);
+    const int nch = sh.nch;
+    PropArgs<T> pa;
+    std::shared_ptr<DevBuf> zt;
+    if ((rc = prop_args<T>(ctx, g, grid, L, sh, thr, st, &pa, &zt))) return rc;
+    if (sh.mfma)
+        for (int i = 0; i < nb; ++i)
+            if ((rc = ensure_kexp(media[i]))) return rc;
     const size_t szW = (size_t)N * K, szPart = (size_t)nch * N * K;
     HIP_TRY(ctx->ws_W.alloc(szW * sizeof(T) * ns));
-    HIP_TRY(ctx->ws_Wp.alloc(szW * sizeof(T) * ns));
+    HIP_TRY(ctx->ws_Wp.alloc(sh.wp * sizeof(T) * ns));
     HIP_TRY(ctx->ws_part.alloc(szPart * sizeof(T) * ns));
     HIP_TRY(ctx->ws_pix.alloc((size_t)kPixBufs * P * sizeof(TA) * ns));
     HIP_TRY(ctx->ws_red.alloc((size_t)2 * sizeof(TA) * ns));
@@ -835,9 +998,10 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
             const int q = i * hv + hh;
             SolveDev<T, TA> &s = sv[q];
             s.W = ctx->ws_W.as<T>() + szW * q;
-            s.Wp = ctx->ws_Wp.as<T>() + szW * q;
+            s.Wp = ctx->ws_Wp.as<T>() + sh.wp * q;
             s.part = ctx->ws_part.as<T>() + szPart * q;
             s.ktab = sizeof(T) == 4 ? (const T *)m->ktab_f.p : (const T *)m->ktab_d.p;
+            s.kexp = m->kexp.as<unsigned char>();
             s.mut = sizeof(T) == 4 ? (const T *)m->mut_f.p : (const T *)m->mut_d.p;
             s.mus = sizeof(T) == 4 ? (const T *)m->mus_f.p : (const T *)m->mus_d.p;
             s.g = T(m->g);
@@ -946,11 +1110,6 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
         }
     }
 
-    PropArgs<T> pa;
-    pa.g = g;
-    pa.nchunk = nch;
-    pa.chunk_len = clen;
-    pa.thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
     CombArgs<T, TA> ca;
     std::memset(&ca, 0, sizeof ca);
     ca.g = g;
@@ -994,6 +1153,35 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
             LaunchTimer tm(ctx, 0);
             HIP_TRY(launch_prop_c<T, TA>(L, path, pa, svd, na, st));
             tm.done(cp_pairs * 2 * na, (flops_dir + 2 * flops_rhs) * na);
+        } else if (sh.mfma) {
+            if constexpr (sizeof(T) == 4) {
+                // groups of any active solves, beams on one medium next to each other (they read
+                // the same path table); the arithmetic of a solve does not depend on its group
+                std::vector<int> order(na);
+                for (int j = 0; j < na; ++j) order[j] = j;
+                std::stable_sort(order.begin(), order.end(),
+                                 [&](int a, int b) { return svact[a].ktab < svact[b].ktab; });
+                svgrp.clear();
+                for (int j : order) svgrp.push_back(svact[j]);
+                HIP_TRY(hipMemcpyAsync(svd_grp, svgrp.data(), sizeof(SolveDev<T, TA>) * na, hipMemcpyHostToDevice, st));
+                {
+                    LaunchTimer tm(ctx, 2);
+                    HIP_TRY(launch_to_pieces<TA>(L, g, svd_grp, na, st));
+                    tm.done();
+                }
+                const std::vector<int> gs = mfma_groups(na, ctx->max_rhs < kMaxNR ? ctx->max_rhs : kMfmaCols);
+                int off = 0;
+                for (size_t i = 0; i < gs.size();) {
+                    size_t e = i;
+                    while (e < gs.size() && gs[e] == gs[i]) ++e;
+                    const int k = gs[i], ng = (int)(e - i);
+                    LaunchTimer tm(ctx, 0, std::min(k, kMaxNR));
+                    HIP_TRY(launch_prop_mfma<TA>(L, k, pa, svd_grp + off, ng, st));
+                    tm.done(cp_pairs * k * ng, (flops_dir + k * flops_rhs) * ng);
+                    off += k * ng;
+                    i = e;
+                }
+            }
         } else if (!multi) {
             LaunchTimer tm(ctx, 0, 1);
             HIP_TRY(launch_prop<T, TA>(L, path, 1, pa, svd, na, st));
@@ -1407,9 +1595,16 @@ extern "C" long long rte_solve_footprint(const rte_grid *grid, const rte_params 
     const long long K = (params->L + 1) * (params->L + 1);
     const long long es = params->precision == RTE_PREC_FP64 ? 8 : 4;
     const long long N = g.N;
-    const int nch = pick_chunks(g.nblk, 1, g.N);
+    // the larger of the shapes that solves of this grid and order take; the 1/64 of a path table
+    // that the matrix cores' exponents take, and the Z table that a grid's solves share, not counted
+    PropShape sh = prop_shape<float>(g, params->L, RTE_PATH_MARCH, false);
+    if (params->precision != RTE_PREC_FP64) {
+        const PropShape m = prop_shape<float>(g, params->L, RTE_PATH_CACHED, false);
+        sh.nch = std::max(sh.nch, m.nch);
+        sh.wp = std::max(sh.wp, m.wp);
+    }
     long long bytes = N * 8 * 3 + N * 4 * 2;             // maps
-    bytes += N * K * es * (2 + nch);                      // W, W in the monomial basis, partials
+    bytes += N * K * es * (1 + sh.nch) + (long long)sh.wp * es;  // W, partials, the propagation's copy of W
     bytes += (long long)grid->nx * grid->ny * kPixBufs * 8 + 64; // pixel buffers
     if (path_mode == RTE_PATH_CACHED) bytes += N * (long long)g.npad * es;
     return bytes;
@@ -1431,8 +1626,9 @@ struct AdjointRun {
     GridDev<T> g{};
     Scales sc{};
     BeamDev bd{};
-    PropArgs<T> pa{};
-    CombArgs<T, TA> ca{};
+    PropArgs<T> pa{}, paf{};  // of the adjoint, of the forward series
+    std::shared_ptr<DevBuf> zt;
+    CombArgs<T, TA> ca{};  // of the forward series
     double coefE[kMaxL + 1] = {};
     HostSolve h{};
     SolveDev<T, TA> sv{};
@@ -1474,10 +1670,12 @@ struct AdjointRun {
         clen = (N + nch0 - 1) / nch0;
         nch = (N + clen - 1) / clen;
         F = (size_t)N * K;
+        const PropShape sh = prop_shape<T>(g, L, RTE_PATH_CACHED, false);  // the forward series'
+        if (sh.mfma && (rc = ensure_kexp(m))) return rc;
         HIP_TRY(dW.alloc(F * sizeof(T)));
-        HIP_TRY(dWp.alloc(F * sizeof(T)));
+        HIP_TRY(dWp.alloc(sh.wp * sizeof(T)));
         HIP_TRY(dS0.alloc(F * sizeof(T)));
-        HIP_TRY(dPart.alloc((size_t)nch * F * sizeof(T)));
+        HIP_TRY(dPart.alloc((size_t)std::max(nch, sh.nch) * F * sizeof(T)));
         HIP_TRY(dPix.alloc((size_t)kPixBufs * P * sizeof(TA)));
         HIP_TRY(dRed.alloc(2 * sizeof(TA)));
         HIP_TRY(dSv.alloc(sizeof(SolveDev<T, TA>)));
@@ -1499,6 +1697,7 @@ struct AdjointRun {
         sv.Wp = dWp.as<T>();
         sv.part = dPart.as<T>();
         sv.ktab = sizeof(T) == 4 ? (const T *)m->ktab_f.p : (const T *)m->ktab_d.p;
+        sv.kexp = m->kexp.as<unsigned char>();
         sv.mut = sizeof(T) == 4 ? (const T *)m->mut_f.p : (const T *)m->mut_d.p;
         sv.mus = sizeof(T) == 4 ? (const T *)m->mus_f.p : (const T *)m->mus_d.p;
         sv.g = T(m->g);
@@ -1528,9 +1727,10 @@ struct AdjointRun {
         pa.nchunk = nch;
         pa.chunk_len = clen;
         pa.thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
+        if ((rc = prop_args<T>(ctx, g, grid, L, sh, thr, st, &paf, &zt))) return rc;
         std::memset(&ca, 0, sizeof ca);
         ca.g = g;
-        ca.nchunk = nch;
+        ca.nchunk = sh.nch;
         ca.mom = sizeof(TA) == 4 ? (const TA *)mom->mf.p : (const TA *)mom->md.p;
         ca.momT = sizeof(T) == 4 ? (const T *)mom->mf.p : (const T *)mom->md.p;
         ca.self_scale = TA((M_PI / kAngRes) * (2.0 * M_PI / kAngRes) / dV);
@@ -1556,7 +1756,7 @@ struct AdjointRun {
                 sv.aw_store = ckpt[q]->as<TA>();
             }
             HIP_TRY(hipMemcpyAsync(svd, &sv, sizeof sv, hipMemcpyHostToDevice, st));
-            HIP_TRY(launch_prop<T, TA>(L, RTE_PATH_CACHED, 1, pa, svd, 1, st));
+            HIP_TRY(launch_prop<T, TA>(L, RTE_PATH_CACHED, 1, paf, svd, 1, st));
             HIP_TRY(launch_combine<T, TA>(L, ca, svd, 1, st));
             HIP_TRY(launch_bottom<T, TA>(P, svd, 1, st));
             HIP_TRY(hipMemcpyAsync(red, dRed.p, sizeof red, hipMemcpyDeviceToHost, st));
@@ -1682,7 +1882,7 @@ struct AdjointRun {
                     s2.mode = 3;
                     s2.aw_store = seg[qq - jc]->as<TA>();
                     HIP_TRY(hipMemcpyAsync(svd, &s2, sizeof s2, hipMemcpyHostToDevice, st));
-                    HIP_TRY(launch_prop<T, TA>(L, RTE_PATH_CACHED, 1, pa, svd, 1, st));
+                    HIP_TRY(launch_prop<T, TA>(L, RTE_PATH_CACHED, 1, paf, svd, 1, st));
                     HIP_TRY(launch_combine<T, TA>(L, ca, svd, 1, st));
                 }
             }
@@ -2081,14 +2281,17 @@ static int propagate_impl(rte_ctx *ctx, rte_medium *m, int L, double prop_thresh
     int rc;
     if ((rc = get_moments(ctx, L, dx, dy, dz, &mom))) return rc;
     if (path == RTE_PATH_CACHED && (rc = ensure_ktab<T>(m, thr))) return rc;
-    const int nch0 = pick_chunks(g.nblk, 1, N);
-    const int clen = (N + nch0 - 1) / nch0;
-    const int nch = (N + clen - 1) / clen;
+    const PropShape sh = prop_shape<T>(g, L, path, false);
+    const int nch = sh.nch;
+    PropArgs<T> pa;
+    std::shared_ptr<DevBuf> zt;
+    if ((rc = prop_args<T>(ctx, g, grid, L, sh, thr, st, &pa, &zt))) return rc;
+    if (sh.mfma && (rc = ensure_kexp(m))) return rc;
     DevBuf dIn, dW, dWp, dPart, dAW, dOut, dSv;
     const size_t nio = (size_t)K * N * (cplx ? 2 : 1);
     HIP_TRY(dIn.alloc(nio * 8));
     HIP_TRY(dW.alloc((size_t)K * N * sizeof(T)));
-    HIP_TRY(dWp.alloc((size_t)K * N * sizeof(T)));
+    HIP_TRY(dWp.alloc(sh.wp * sizeof(T)));
     HIP_TRY(dPart.alloc((size_t)nch * N * K * sizeof(T)));
     HIP_TRY(dAW.alloc((size_t)K * N * sizeof(TA)));
     HIP_TRY(dOut.alloc(nio * 8));
@@ -2105,15 +2308,11 @@ static int propagate_impl(rte_ctx *ctx, rte_medium *m, int L, double prop_thresh
     s.Wp = dWp.as<T>();
     s.part = dPart.as<T>();
     s.ktab = sizeof(T) == 4 ? (const T *)m->ktab_f.p : (const T *)m->ktab_d.p;
+    s.kexp = m->kexp.as<unsigned char>();
     s.mut = sizeof(T) == 4 ? (const T *)m->mut_f.p : (const T *)m->mut_d.p;
     s.mus = sizeof(T) == 4 ? (const T *)m->mus_f.p : (const T *)m->mus_d.p;
     s.g = T(m->g);
     HIP_TRY(hipMemcpyAsync(dSv.p, &s, sizeof s, hipMemcpyHostToDevice, st));
-    PropArgs<T> pa;
-    pa.g = g;
-    pa.nchunk = nch;
-    pa.chunk_len = clen;
-    pa.thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
     HIP_TRY(launch_prop<T, TA>(L, path, 1, pa, dSv.as<SolveDev<T, TA>>(), 1, st));
     CombArgs<T, TA> ca;
     std::memset(&ca, 0, sizeof ca);
@@ -2485,8 +2684,6 @@ extern "C" int rte_path_integrals(rte_ctx *ctx, const rte_grid *grid, const rte_
 #include <atomic>
 #include <condition_variable>
 #include <deque>
-#include <list>
-#include <mutex>
 #include <thread>
 
 namespace {
@@ -2518,12 +2715,12 @@ struct SlotBase {
     ServReq *r = nullptr;  // null: idle
     int idx = 0;           // row of the bucket's reduction and image arrays
     long long bytes = 0;
-    DevBuf mua, mus, mutd, mutf, musf, ktab, W, Wp, part, pix;
+    DevBuf mua, mus, mutd, mutf, musf, ktab, kexp, W, Wp, part, pix;
     HostSolve h{};
     bool fresh = false, ran = false;
     void free_memory()
     {
-        for (DevBuf *b : {&mua, &mus, &mutd, &mutf, &musf, &ktab, &W, &Wp, &part, &pix}) b->release();
+        for (DevBuf *b : {&mua, &mus, &mutd, &mutf, &musf, &ktab, &kexp, &W, &Wp, &part, &pix}) b->release();
         bytes = 0;
     }
 };
@@ -2573,7 +2770,9 @@ struct Bucket : BucketBase {
     rte_ctx *ctx = nullptr;
     rte_grid grid{};
     rte_params p{};
-    int L = 0, K = 0, N = 0, P = 0, nch = 0, clen = 0, max_terms = 0;
+    int L = 0, K = 0, N = 0, P = 0, max_terms = 0;
+    PropShape sh;
+    std::shared_ptr<DevBuf> zt;
     double dx = 0, dy = 0, dz = 0, thr = -1;
     GridDev<T> g{};
     Scales sc{};
@@ -2602,18 +2801,12 @@ struct Bucket : BucketBase {
         thr = p.prop_thresh > 0 ? p.prop_thresh : -1.0;
         max_terms = p.max_terms > 0 ? p.max_terms : 1000;
         slot_bytes = rte_solve_footprint(&grid, &p, p.path_mode);
-        // the same source chunking as rte_solve_media: it depends on the grid only
-        const int nch0 = pick_chunks(g.nblk, 1, N);
-        clen = (N + nch0 - 1) / nch0;
-        nch = (N + clen - 1) / clen;
+        // the same source chunking as rte_solve_media
+        sh = prop_shape<T>(g, L, p.path_mode, false);
         sc = make_scales(L);
-        pa.g = g;
-        pa.nchunk = nch;
-        pa.chunk_len = clen;
-        pa.thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
         std::memset(&ca, 0, sizeof ca);
         ca.g = g;
-        ca.nchunk = nch;
+        ca.nchunk = sh.nch;
         ca.op = 0;
         ca.mom = sizeof(TA) == 4 ? (const TA *)mom->mf.p : (const TA *)mom->md.p;
         ca.momT = sizeof(T) == 4 ? (const T *)mom->mf.p : (const T *)mom->md.p;
@@ -2637,6 +2830,7 @@ struct Bucket : BucketBase {
             init_err = RTE_E_DEVICE;
             return;
         }
+        if ((init_err = prop_args<T>(ctx, g, grid, L, sh, thr, stream, &pa, &zt))) return;
         const size_t svb = sizeof(SolveDev<T, TA>) * cap;
         if (hipEventCreateWithFlags(&ev_step, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&ev_drain, hipEventDisableTiming) != hipSuccess) {
@@ -2677,7 +2871,8 @@ struct Bucket : BucketBase {
         const bool cached = p.path_mode == RTE_PATH_CACHED;
         if (s.mua.alloc(n * 8) || s.mus.alloc(n * 8) || s.mutd.alloc(n * 8) || s.mutf.alloc(n * 4) ||
             s.musf.alloc(n * 4) || (cached && s.ktab.alloc((size_t)N * g.npad * sizeof(T))) ||
-            s.W.alloc(F * sizeof(T)) || s.Wp.alloc(F * sizeof(T)) || s.part.alloc((size_t)nch * F * sizeof(T)) ||
+            (sh.mfma && s.kexp.alloc(kexp_bytes(make_grid<float>(grid)))) ||
+            s.W.alloc(F * sizeof(T)) || s.Wp.alloc(sh.wp * sizeof(T)) || s.part.alloc((size_t)sh.nch * F * sizeof(T)) ||
             s.pix.alloc((size_t)kPixBufs * P * sizeof(TA))) {
             s.free_memory();
             return fail(RTE_E_NOMEM, "server: device memory for a %dx%dx%d L=%d solve", grid.nx, grid.ny, grid.nz, L);
@@ -2699,6 +2894,9 @@ struct Bucket : BucketBase {
         const T *mut = sizeof(T) == 4 ? (const T *)s.mutf.p : (const T *)s.mutd.p;
         if (p.path_mode == RTE_PATH_CACHED)
             HIP_TRY(launch_ktab<T>(g, pa.thr2, mut, s.ktab.template as<T>(), stream));
+        if constexpr (sizeof(T) == 4)
+            if (sh.mfma)
+                HIP_TRY(launch_kexp(g, s.ktab.template as<float>(), s.kexp.template as<unsigned char>(), stream));
         const size_t F = (size_t)N * K;
         HIP_TRY(launch_fill<T>(s.W.template as<T>(), F, T(0), stream));
         SolveDev<T, TA> &v = sv[s.idx];
@@ -2707,6 +2905,7 @@ struct Bucket : BucketBase {
         v.Wp = s.Wp.template as<T>();
         v.part = s.part.template as<T>();
         v.ktab = p.path_mode == RTE_PATH_CACHED ? s.ktab.template as<T>() : nullptr;
+        v.kexp = s.kexp.template as<unsigned char>();
         v.mut = mut;
         v.mus = sizeof(T) == 4 ? (const T *)s.musf.p : (const T *)s.mus.p;
         v.g = T(r->g);
@@ -2767,9 +2966,19 @@ struct Bucket : BucketBase {
                 // resident solves in pairs across media on the mixed cached path (they
                 // share the pair geometry, each reads its own table), the odd one alone
                 hipError_t e = hipSuccess;
-                const int npair = (sizeof(T) == 4 && sizeof(TA) == 8 && p.path_mode == RTE_PATH_CACHED) ? na / 2 : 0;
+                int done = 0;
+                if constexpr (sizeof(T) == 4) {
+                    if (sh.mfma) {
+                        e = launch_to_pieces<TA>(L, g, d, na, stream);
+                        for (int k : mfma_groups(na, kMfmaCols)) {
+                            if (e == hipSuccess) e = launch_prop_mfma<TA>(L, k, pa, d + done, 1, stream);
+                            done += k;
+                        }
+                    }
+                }
+                const int npair = done ? 0 : (sizeof(T) == 4 && sizeof(TA) == 8 && p.path_mode == RTE_PATH_CACHED) ? na / 2 : 0;
                 if (npair) e = launch_prop_sep<T, TA>(L, 2, pa, d, npair, stream);
-                if (e == hipSuccess && na > 2 * npair)
+                if (e == hipSuccess && !done && na > 2 * npair)
                     e = launch_prop<T, TA>(L, p.path_mode, 1, pa, d + 2 * npair, na - 2 * npair, stream);
                 if (e == hipSuccess) e = launch_combine<T, TA>(L, ca, d, na, stream);
                 if (e == hipSuccess) e = launch_bottom<T, TA>(P, d, na, stream);

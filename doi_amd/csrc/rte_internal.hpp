@@ -56,6 +56,7 @@ struct SolveDev {
     T *Wp;             // [N][K] the same in the propagation's z-power basis, written by each launch
     T *part;           // [nchunk][N][K] partial pair sums
     const T *ktab;     // [N][npad] e^{-tau}/r^2 per (source, destination slot), cached mode
+    const unsigned char *kexp;  // [slab][npad] exponents of the path table (rte_mfma.hip), if it is used there
     const T *mut;      // [N] mu_t
     const T *mus;      // [N] mu_s
     T g;               // anisotropy
@@ -80,6 +81,22 @@ struct PropArgs {
     GridDev<T> g;
     int nchunk, chunk_len;
     T thr2;  // prop_thresh^2; pairs with r^2 >= thr2 are dropped
+    // the matrix-core propagation (rte_mfma.hip, whose chunks are of source brick rows): its
+    // Z table; nullptr for k_prop
+    const unsigned char *zt = nullptr;
+};
+
+// arguments of k_prop_mfma
+constexpr int kMfmaThreads = 512;  // 8 waves, 2 per SIMD
+constexpr int kMfmaCols = 16;      // columns of its products: right-hand sides x translations
+struct MfmaArgs {
+    GridDev<float> g;
+    const unsigned char *zt;   // [2 nz - 1][8 by - 1][nxt] rows of Z pieces
+    float thr2;
+    int nr, ntx, ntz;          // right-hand sides of a group, translations by bricks (nr ntx ntz <= 16)
+    int nxg;                   // units along x
+    int nchunk;                // chunks of source brick rows
+    int nxt;
 };
 
 // combine launch: A.op = 1 writes A W to aw_out; otherwise the per-solve mode
@@ -128,6 +145,20 @@ hipError_t launch_prop_sep(int L, int nr, const PropArgs<T> &A, const SolveDev<T
 template <typename T, typename TA>
 hipError_t launch_prop_c(int L, int path, const PropArgs<T> &A, const SolveDev<T, TA> *sv, int ncomplex,
                          hipStream_t st);
+// matrix-core propagation (rte_mfma.hip), A.zt set: ngroups * nr solves on any media of one
+// grid, their W first brought into pieces; each solve's Wp holds mfma_wp_bytes
+size_t mfma_wp_bytes(int L, const GridDev<float> &g);
+double mfma_translations(const GridDev<float> &g, int nr, int *ntx, int *ntz);
+size_t mfma_ztab_bytes(int L, const GridDev<float> &g);
+// the exponents of a path table
+size_t kexp_bytes(const GridDev<float> &g);
+hipError_t launch_kexp(const GridDev<float> &g, const float *ktab, unsigned char *kexp, hipStream_t st);
+hipError_t launch_ztab(int L, const GridDev<float> &g, double dx, double dy, double dz, unsigned char *zt, hipStream_t st);
+template <typename TA>
+hipError_t launch_to_pieces(int L, const GridDev<float> &g, const SolveDev<float, TA> *sv, int nsolve, hipStream_t st);
+template <typename TA>
+hipError_t launch_prop_mfma(int L, int nr, const PropArgs<float> &A, const SolveDev<float, TA> *sv, int ngroups,
+                            hipStream_t st);
 template <typename T>
 hipError_t launch_ktab(const GridDev<T> &g, T thr2, const T *mut, T *ktab, hipStream_t st);
 template <typename T, typename TA>

@@ -1271,6 +1271,12 @@ template <typename T, typename TA>
 hipError_t launch_prop(int L, int path, int nr, const PropArgs<T> &A, const SolveDev<T, TA> *sv, int ngroups,
                        hipStream_t st)
 {
+    if constexpr (sizeof(T) == 4) {
+        if (A.zt && path == 0) {
+            const hipError_t e = launch_to_pieces<TA>(L, A.g, sv, ngroups * nr, st);
+            return e != hipSuccess ? e : launch_prop_mfma<TA>(L, nr, A, sv, ngroups, st);
+        }
+    }
     dim3 grid((A.g.nblk + kPropWaves - 1) / kPropWaves, A.nchunk, ngroups), block(kWave * kPropWaves);
     // several right-hand sides per group only on the mixed-precision cached path
     constexpr bool multi = sizeof(T) == 4 && sizeof(TA) == 8;

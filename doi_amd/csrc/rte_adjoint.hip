@@ -325,63 +325,114 @@ __global__ void k_make_wq(GridDev<T> g, Scales sc, TA gan, const T *mus, const T
 // centres crosses the same voxels with the same Siddon lengths both ways (the
 // crossings alpha = (j + 1/2)/n mirror into each other; only zero-length
 // segments at exact ties may fall in different voxels), so the pair weights of
-// (d, s) and (s, d) are added and the ray is marched once.  A wave owns a
-// brick pair (bd, bs), bs <= bd (the path table's tiling), lane = destination
-// d in bd, and walks the 64 sources of bs; on the diagonal tile only the pairs
-// with slot(s) < slot(d).  grid = ceil(ntiles / waves per block), block =
-// 1024 (LDS accumulator) or 256.
+// (d, s) and (s, d) are added and the ray is marched once.  As in the path table a
+// brick pair is (bs, bs + D), D in the half space z, then y, then x >= 0; on D = 0
+// only the pairs with slot(s) < slot(d).
+// A wave takes M translations of a brick pair, lane = (translation, 64 / M of the
+// destinations), and walks 16 sources of the brick with M steps over its
+// destinations.  With the 64 destinations of one source in a wave (the layout before
+// this) the rays leave the source through the same few voxels, and the atomics on
+// one address are served one after the other, ~110 clocks of the LDS per crossing;
+// translated rays are in different voxels throughout.  24^3 (FP64 sums) before 9.0,
+// now 3.7 ms.
+// A grid whose sums do not fit the LDS goes in slabs of z planes, a y-row of blocks each:
+// a slab's rays (those that reach it) are walked whole and their voxels outside it left
+// out.  (With atomics in memory a gradient at
+// 28^3, L = 5, 8 terms took 506 ms, 32^3 1302, 40^3, L = 3, 5139; in slabs 55, 92 and 310.)  Only where that takes
+// more than kBpSlabs slabs do the atomics go to memory.
+// grid = (at most the resident blocks, slabs); unit u (translation group, D, 16 of the
+// source brick's 64 voxels) belongs to block u mod grid, whose waves share its units.
 // ---------------------------------------------------------------------------
-template <typename T, typename TA, bool LDS>
-__global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, int ntiles, T thr2, const T *pairbuf,
+constexpr int kBpSlabs = 16;
+struct BpPlan {
+    int py, pz;      // pitches of y and z in the accumulator (elements)
+    int zs;          // z planes of a slab
+    int nD, nunits;
+    int next;        // where in LDS the block's unit counter lies (bytes), -1: no room
+};
+
+// MEM 0: sums in memory; 1: in LDS; 2: in LDS by slabs
+template <typename T, typename TA, int MEM, int M>
+__global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, BpPlan p, T thr2, const T *__restrict__ pairbuf,
                                                           TA scale, TA *gt)
 {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     TA *sacc = reinterpret_cast<TA *>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    if constexpr (LDS) {
-        for (int i = tid; i < g.N; i += blockDim.x) sacc[i] = TA(0);
-        __syncthreads();
-    }
-    const int tile = blockIdx.x * (blockDim.x / kWave) + tid / kWave;
-    if (tile < ntiles) {
-        int bd = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
-        while (bd > 0 && bd * (bd + 1) / 2 > tile) --bd;
-        while ((bd + 1) * (bd + 2) / 2 <= tile) ++bd;
-        const int bs = tile - bd * (bd + 1) / 2;
-        int di, dj, dk;
-        lane_dest(g, bd, lane, di, dj, dk);
-        const bool dvalid = di < g.nx && dj < g.ny && dk < g.nz;
-        const int cdi = min(di, g.nx - 1), cdj = min(dj, g.ny - 1), cdk = min(dk, g.nz - 1);
-        const int nxy = g.nx * g.ny;
-        const int dslot = bd * kWave + lane;
-        const int dlin = cdi + g.nx * cdj + nxy * cdk;
-        const int bxi = bs % g.bx, byi = (bs / g.bx) % g.by, bzi = bs / (g.bx * g.by);
-        for (int q = 0; q < kWave; ++q) {
-            const int si = bxi * kBrick + (q & 3), sj = byi * kBrick + ((q >> 2) & 3), sk = bzi * kBrick + (q >> 4);
-            if (si >= g.nx || sj >= g.ny || sk >= g.nz) continue;  // wave-uniform
-            const int sslot = bs * kWave + q;
-            const int ix = cdi - si, iy = cdj - sj, iz = cdk - sk;
-            const T ddx = T(ix) * g.dx, ddy = T(iy) * g.dy, ddz = T(iz) * g.dz;
-            const T r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-            const bool self = (ix == 0) && (iy == 0) && (iz == 0);
-            const bool once = bs != bd || sslot < dslot;
-            if (!(dvalid && !self && once && r2 < thr2)) continue;
-            const int slin = si + g.nx * sj + nxy * sk;
-            const TA w = TA(pairbuf[(size_t)slin * g.npad + dslot]) + TA(pairbuf[(size_t)dlin * g.npad + sslot]);
+    int *next = reinterpret_cast<int *>(smem_raw + p.next);
+    constexpr int ND = kWave / M;                   // destinations side by side
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), m = lane / ND, sub = lane % ND;
+    const int nxy = g.nx * g.ny;
+    constexpr bool LDS = MEM != 0;
+    const int z0 = MEM == 2 ? blockIdx.y * p.zs : 0, z1 = MEM == 2 ? min(z0 + p.zs, g.nz) : g.nz;
+    const int lo = z0 * p.pz, size = (z1 - z0) * p.pz;
+    if constexpr (LDS)
+        for (int i = tid; i < size; i += blockDim.x) sacc[i] = TA(0);
+    if (p.next >= 0 && tid == 0) *next = 0;
+    __syncthreads();
+    const int ex = 2 * g.bx - 1, ey = 2 * g.by - 1;
+    for (int own = tid / kWave;; own += blockDim.x / kWave) {
+        // the block's next unit (in a fixed order where the accumulator leaves no room for a counter)
+        if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
+        const int u = blockIdx.x + gridDim.x * __builtin_amdgcn_readfirstlane(own);
+        if (u >= p.nunits) break;
+        const int slab = u & 3, f = (u >> 2) % p.nD + p.nD - 1, first = (u >> 2) / p.nD * M;
+        const int Dx = f % ex - (g.bx - 1), Dy = (f / ex) % ey - (g.by - 1), Dz = f / (ex * ey) - (g.bz - 1);
+        const int cx = g.bx - abs(Dx), cy = g.by - abs(Dy), cnt = cx * cy * (g.bz - abs(Dz));
+        if (first >= cnt) continue;
+        const bool other = (Dx | Dy | Dz) != 0, live = first + m < cnt;
+        // this lane's source brick
+        const int t = min(first + m, cnt - 1);
+        const int bx0 = t % cx + max(0, -Dx), by0 = (t / cx) % cy + max(0, -Dy), bz0 = t / (cx * cy) + max(0, -Dz);
+        const int bs = bx0 + g.bx * (by0 + g.by * bz0), bd = bs + Dx + g.bx * (Dy + g.by * Dz);
+        // pair it = source 16 slab + it / M of the brick, destination slot (it % M) ND + sub
+        struct Pair { int ix, iy, iz, v; T r2, w0, w1; };
+        auto load = [&](int it) {
+            const int q = slab * 16 + it / M, j = it % M * ND + sub;
+            const int sx = q & 3, sy = (q >> 2) & 3, sz = q >> 4, lx = j & 3, ly = (j >> 2) & 3, lz = j >> 4;
+            const int x = bx0 * kBrick + sx, y = by0 * kBrick + sy, z = bz0 * kBrick + sz;
+            Pair P;
+            P.ix = Dx * kBrick + lx - sx;
+            P.iy = Dy * kBrick + ly - sy;
+            P.iz = Dz * kBrick + lz - sz;
+            const int X = x + P.ix, Y = y + P.iy, Z = z + P.iz;
+            const T ddx = T(P.ix) * g.dx, ddy = T(P.iy) * g.dy, ddz = T(P.iz) * g.dz;
+            P.r2 = sum_squares(ddx, ddy, ddz);
+            const bool ok = live && x < g.nx && y < g.ny && z < g.nz && X < g.nx && Y < g.ny && Z < g.nz &&
+                            (other || q < j) && P.r2 < thr2 && (MEM != 2 || (max(z, Z) >= z0 && min(z, Z) < z1));
+            P.v = LDS ? x + p.py * y + p.pz * z : x + g.nx * y + nxy * z;
+            P.w0 = P.w1 = T(0);
+            if (ok) {
+                P.w0 = pairbuf[(size_t)(x + g.nx * y + nxy * z) * g.npad + bd * kWave + j];
+                P.w1 = pairbuf[(size_t)(X + g.nx * Y + nxy * Z) * g.npad + bs * kWave + q];
+            }
+            return P;
+        };
+        Pair nx = load(0);
+        for (int it = 0; it < 16 * M; ++it) {
+            const Pair P = nx;
+            if (it + 1 < 16 * M) nx = load(it + 1);  // the next pair's weights under this one's march
+            const TA w = TA(P.w0) + TA(P.w1);
             if (w == TA(0)) continue;
             const TA sw = scale * w;
-            march_visit<T>(slin, ix, iy, iz, g.nx, nxy, sqrt(r2), [&](int v, T len) {
-                if constexpr (LDS)
+            const T r = sqrt(P.r2);
+            march_visit<T>(P.v, P.ix, P.iy, P.iz, LDS ? p.py : g.nx, LDS ? p.pz : nxy, r, [&](int v, T len) {
+                if constexpr (MEM == 2) {
+                    if ((unsigned)(v - lo) < (unsigned)size) atomicAdd(&sacc[v - lo], sw * TA(len));
+                } else if constexpr (LDS) {
                     atomicAdd(&sacc[v], sw * TA(len));
-                else
+                } else {
                     atomicAdd(&gt[v], sw * TA(len));
+                }
             });
         }
     }
     if constexpr (LDS) {
         __syncthreads();
-        for (int i = tid; i < g.N; i += blockDim.x)
-            if (sacc[i] != TA(0)) atomicAdd(&gt[i], sacc[i]);
+        for (int i = z0 * nxy + tid; i < z1 * nxy; i += blockDim.x) {
+            const int x = i % g.nx, y = (i / g.nx) % g.ny, z = i / nxy;
+            const TA a = sacc[x + p.py * y + p.pz * z - lo];
+            if (a != TA(0)) atomicAdd(&gt[i], a);
+        }
     }
 }
 
@@ -426,7 +477,7 @@ __global__ __launch_bounds__(1024) void k_backproject_blocks(GridDev<T> g, int n
             const int sslot = bs * kWave + q;
             const int ix = cdi - si, iy = cdj - sj, iz = cdk - sk;
             const T ddx = T(ix) * g.dx, ddy = T(iy) * g.dy, ddz = T(iz) * g.dz;
-            const T r2 = ddx * ddx + ddy * ddy + ddz * ddz;
+            const T r2 = sum_squares(ddx, ddy, ddz);
             const bool self = (ix == 0) && (iy == 0) && (iz == 0);
             const bool once = bs != bd || sslot < dslot;
             if (!(dvalid && !self && once && r2 < thr2)) continue;
@@ -646,39 +697,64 @@ hipError_t launch_make_wq(int L, const GridDev<T> &g, const Scales &sc, TA gan, 
     return hipGetLastError();
 }
 
-template <typename T, typename TA>
-hipError_t launch_backproject(const GridDev<T> &g, int nchunk, int chunk_len, T thr2, const T *pairbuf, TA scale,
-                              TA *gt, hipStream_t st)
+template <typename T, typename TA, int MEM, int M>
+static hipError_t launch_bp_as(const GridDev<T> &g, BpPlan p, size_t lds, int cus, T thr2, const T *pairbuf, TA scale,
+                               TA *gt, hipStream_t st)
 {
-    static int lds_max = -1;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_backproject_sym<T, TA, MEM, M>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    // a large accumulator leaves room for one block per CU: make it 16 waves
+    const int threads = lds > 64 * 1024 ? 1024 : 256, waves = threads / kWave;
+    p.nunits = p.nD * ((g.nblk + M - 1) / M) * 4;
+    const int blocks = min((p.nunits + waves - 1) / waves, cus * (1024 / threads));
+    const int slabs = MEM == 2 ? (g.nz + p.zs - 1) / p.zs : 1;
+    hipLaunchKernelGGL((k_backproject_sym<T, TA, MEM, M>), dim3(blocks, slabs), dim3(threads), lds, st, g, p, thr2, pairbuf,
+                       scale, gt);
+    return hipGetLastError();
+}
+
+template <typename T, typename TA>
+hipError_t launch_backproject(const GridDev<T> &g, T thr2, const T *pairbuf, TA scale, TA *gt, hipStream_t st)
+{
+    static int lds_max = -1, cus = 0;
     if (lds_max < 0) {
         int dev = 0, v = 0;
         hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
         if (e != hipSuccess) return e;
         lds_max = v;
     }
-    const size_t lds = (size_t)g.N * sizeof(TA);
-    const int ntiles = g.nblk * (g.nblk + 1) / 2;
-    (void)nchunk;
-    (void)chunk_len;
-    if (lds <= (size_t)lds_max) {
-        // a large accumulator leaves room for one block per CU: make it 16 waves
-        const int threads = lds > 64 * 1024 ? 1024 : 256;
-        if (lds > 64 * 1024) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_backproject_sym<T, TA, true>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        const int waves = threads / kWave;
-        hipLaunchKernelGGL((k_backproject_sym<T, TA, true>), dim3((ntiles + waves - 1) / waves), dim3(threads), lds,
-                           st, g, ntiles, thr2, pairbuf, scale, gt);
-    } else {
-        constexpr int threads = 256, waves = threads / kWave;
-        hipLaunchKernelGGL((k_backproject_sym<T, TA, false>), dim3((ntiles + waves - 1) / waves), dim3(threads), 0,
-                           st, g, ntiles, thr2, pairbuf, scale, gt);
+    // odd pitches (the translations' voxels in different banks) where that fits
+    BpPlan p{};
+    size_t lds = 0;
+    auto fits = [&](int py, int pz, int slabs) {
+        p.py = py;
+        p.pz = pz;
+        p.zs = (g.nz + slabs - 1) / slabs;
+        const size_t acc = ((size_t)pz * p.zs * sizeof(TA) + 15) / 16 * 16;
+        p.next = acc + 16 <= (size_t)lds_max ? (int)acc : -1;
+        lds = p.next >= 0 ? acc + 16 : acc;
+        return lds <= (size_t)lds_max;
+    };
+    int mem = 0;
+    for (int n = 1; n <= kBpSlabs && n <= g.nz && !mem; ++n)
+        if (fits(g.nx | 1, (g.nx | 1) * g.ny | 1, n) || fits(g.nx, g.nx * g.ny, n)) mem = n == 1 ? 1 : 2;
+    if (!mem) {
+        p.next = 0;
+        lds = 16;
     }
-    return hipGetLastError();
+    p.nD = ((2 * g.bx - 1) * (2 * g.by - 1) * (2 * g.bz - 1) + 1) / 2;
+    // 16 translations where most brick displacements have that many, else 4
+    const bool many = g.nblk >= 64;
+#define RTE_BP(MEM)                                                                              \
+    (many ? launch_bp_as<T, TA, MEM, 16>(g, p, lds, cus, thr2, pairbuf, scale, gt, st)           \
+          : launch_bp_as<T, TA, MEM, 4>(g, p, lds, cus, thr2, pairbuf, scale, gt, st))
+    return mem == 1 ? RTE_BP(1) : mem == 2 ? RTE_BP(2) : RTE_BP(0);
+#undef RTE_BP
 }
 
 template <typename T, typename TA>
@@ -764,9 +840,9 @@ template hipError_t launch_make_wq<float, double>(int, const GridDev<float> &, c
                                                   const float *, const double *, float *, hipStream_t);
 template hipError_t launch_make_wq<double, double>(int, const GridDev<double> &, const Scales &, double,
                                                    const double *, const double *, double *, hipStream_t);
-template hipError_t launch_backproject<float, double>(const GridDev<float> &, int, int, float, const float *,
+template hipError_t launch_backproject<float, double>(const GridDev<float> &, float, const float *,
                                                       double, double *, hipStream_t);
-template hipError_t launch_backproject<double, double>(const GridDev<double> &, int, int, double, const double *,
+template hipError_t launch_backproject<double, double>(const GridDev<double> &, double, const double *,
                                                        double, double *, hipStream_t);
 template hipError_t launch_backproject_blocks<float, double>(const GridDev<float> &, float,
                                                              const BlockBp<float, double> &, int, hipStream_t);

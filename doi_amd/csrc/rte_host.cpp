@@ -1928,7 +1928,7 @@ struct AdjointRun {
         }
         for (int c = 0; c < nc; ++c) {
             if (!(blk && blk->used))
-                HIP_TRY(launch_backproject<T, TA>(g, nch, clen, pa.thr2, dPair[c].as<T>(), TA(-dV), dGt[c].as<TA>(),
+                HIP_TRY(launch_backproject<T, TA>(g, pa.thr2, dPair[c].as<T>(), TA(-dV), dGt[c].as<TA>(),
                                                   st));
             HIP_TRY(launch_src_grad<TA>(L, grid.nx, grid.ny, grid.nz, dx, dy, dz, grid.xmin, grid.ymin, m->g, bd,
                                         dLam0[c].as<TA>(), dCot[c].as<TA>(), dGa2[c].as<TA>(), dGs2[c].as<TA>(), st));

@@ -255,8 +255,7 @@ struct BlockBp {
 template <typename T, typename TA>
 hipError_t launch_backproject_blocks(const GridDev<T> &g, T thr2, const BlockBp<T, TA> &B, int nc, hipStream_t st);
 template <typename T, typename TA>
-hipError_t launch_backproject(const GridDev<T> &g, int nchunk, int chunk_len, T thr2, const T *pairbuf, TA scale,
-                              TA *gt, hipStream_t st);
+hipError_t launch_backproject(const GridDev<T> &g, T thr2, const T *pairbuf, TA scale, TA *gt, hipStream_t st);
 template <typename TA>
 hipError_t launch_src_grad(int L, int nx, int ny, int nz, double dx, double dy, double dz, double xmin, double ymin,
                            double gan, const BeamDev &B, const TA *lam0, const TA *cot, TA *ga, TA *gs, hipStream_t st);

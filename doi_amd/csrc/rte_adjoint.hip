@@ -161,118 +161,177 @@ __global__ __launch_bounds__(256) void k_bufs_to_zpow(int N, ZBufs<T> B)
 // ---------------------------------------------------------------------------
 // Per voxel: Lambda_q = A^T xi_q, the self-block and scatter gradient terms,
 // and the next adjoint input xi_{q-1} = eps + D Lambda_q (written over X).
-// grid = ceil(N/64), block = 64.
+// Laid out as k_combine, and bound by the same partials: a thread per (voxel,
+// coefficient) in place of one per voxel, 24^3, L = 5, FP32 143 -> 30 us; a 16^3
+// gradient of 8 terms 4.87 -> 4.20 ms, 9^3 at L = 7 2.83 -> 1.71.
+// The self block S(mu) = self_scale sum_k c_k M_k, c_k = (-mu)^{k-1}/k!, acts on xi
+// (c_k), and on W_q for its mu-derivative (dc_k/dmu): two products with each moment.
+// grid = ceil(N/VB), block = kCombThreads.
 // ---------------------------------------------------------------------------
 template <typename T, typename TA, int L>
-__global__ __launch_bounds__(kWave) void k_adj_combine(AdjCombArgs<T, TA> A)
+__global__ __launch_bounds__(kCombThreads) void k_adj_combine(AdjCombArgs<T, TA> A)
 {
-    constexpr int K = (L + 1) * (L + 1);
+    using Sh = CombShape<L>;
+    constexpr int K = Sh::K, VP = Sh::VP, VPT = Sh::VPT, VB = Sh::VB, NJ = Sh::NJ, NZ = Sh::NZ;
+    constexpr bool f32 = sizeof(T) == 4;
+    __shared__ TA zs[VB * K];               // z-power sums
+    __shared__ TA gp[VB * K], sp[VB * K];   // terms of the mu_t and mu_s gradients; FP64: the self block's sums first
+    __shared__ T xs[VB * K], ws[VB * K];    // xi, W_q
+    __shared__ T cf[2][kNMom][VB];          // c_k, dc_k/dmu
+    __shared__ T ms[f32 ? kNMom * NJ * K : 1];
     const GridDev<T> &g = A.g;
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= g.N) return;
-    TA acc[K], xi[K], w[K];
-#pragma unroll
-    for (int a = 0; a < K; ++a) {
-        const TA sgn = (l_of<L>(a) & 1) ? TA(-1) : TA(1);
-        xi[a] = sgn * TA(A.X[(size_t)v * K + a]) / A.nsc[a];
-        w[a] = TA(A.Wq[(size_t)v * K + a]) / A.nsc[a];
-        acc[a] = TA(0);
-    }
-    for (int c = 0; c < A.nchunk; ++c) {
-        const T *__restrict__ p = A.part + ((size_t)c * g.N + v) * K;
-#pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] += TA(p[a]);
-    }
-    zpow_to_harmonic<TA, L>(acc);
-#pragma unroll
-    for (int a = 0; a < K; ++a) {
-        const TA sgn = (l_of<L>(a) & 1) ? TA(-1) : TA(1);
-        acc[a] = sgn * acc[a] * A.nsc[a];
-    }
-    // self block S(mu) = self_scale sum_k c_k M_k, c_k = (-mu)^{k-1}/k!, and its mu-derivative;
-    // the FP32 path uses the same FP32 entries as the forward combine (S symmetric)
-    TA gself = TA(0);
-    if constexpr (sizeof(T) == 4) {
-        T xt[K], wt[K], st[K];
-#pragma unroll
-        for (int a = 0; a < K; ++a) {
-            xt[a] = T(xi[a]);
-            wt[a] = T(w[a]);
-            st[a] = T(0);
+    const CombTab<L> &tab = kCombTab<L>;
+    const int tid = threadIdx.x, v0 = blockIdx.x * VB;
+    const bool live = tid < VP * K;
+    const int a = tid % K, q0 = tid / K;
+    if constexpr (f32) {
+        for (int q = tid; q < kNMom * NJ * K; q += kCombThreads) {
+            const int aa = q % K, i = (q / K) % NJ, k = q / (K * NJ), b = tab.b[i][aa];
+            ms[q] = b < 0 ? T(0) : A.momT[(size_t)k * K * K + aa * K + b];
         }
-        const T mu = A.mut[v];
-        T coef = T(1), dcoef = T(0), pw = T(1), fact = T(1), gs = T(0);
+    }
+    if (tid < VB) {
+        // c = (-mu)^k/(k+1)!, dc/dmu = -k (-mu)^{k-1}/(k+1)! for moment index k+1; pw = (-mu)^{k-1}
+        const T mu = A.mut[min(v0 + tid, g.N - 1)];
+        T pw = T(1), fact = T(1);
         for (int k = 0; k < kNMom; ++k) {
             fact *= T(k + 1);
-            dcoef = (k == 0) ? T(0) : -T(k) * pw / fact;
+            cf[1][k][tid] = (k == 0) ? T(0) : -T(k) * pw / fact;
             pw = (k == 0) ? T(1) : pw * (-mu);
-            coef = pw / fact;
-            T gk = T(0);
-            self_apply_adj<K>(st, gk, coef, A.momT + (size_t)k * K * K, xt, wt, std::make_integer_sequence<int, K>{});
-            gs += dcoef * gk;
+            cf[0][k][tid] = pw / fact;
+        }
+    }
+    const TA na = A.nsc[live ? a : 0];
+    const TA sgn = (l_of<L>(a) & 1) ? TA(-1) : TA(1);
+    if (live) {
+        const size_t cs = (size_t)g.N * K;
+        size_t e[VPT];
+        TA sum[VPT];
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int v = v0 + i * VP + q0;
+            e[i] = v < g.N ? (size_t)v * K + a : a;  // beyond the grid: voxel 0's, not used
+            xs[i * VP * K + tid] = T(sgn * TA(A.X[e[i]]) / na);
+            ws[i * VP * K + tid] = T(TA(A.Wq[e[i]]) / na);
+            sum[i] = TA(0);
+        }
+        const T *__restrict__ p = A.part;
+#pragma unroll 8
+        for (int c = 0; c < A.nchunk; ++c, p += cs) {
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) sum[i] += TA(p[e[i]]);
         }
 #pragma unroll
-        for (int a = 0; a < K; ++a) acc[a] += A.self_scale * TA(st[a]);
-        gself = TA(gs);
-    } else {
-        const TA mu = TA(A.mut[v]);
-        TA coef = TA(1), dcoef = TA(0), pw = TA(1);  // pw = (-mu)^{k-1}
-        TA fact = TA(1);
-        for (int k = 0; k < kNMom; ++k) {
-            // k here is moment index k+1: c = (-mu)^k/(k+1)!, dc/dmu = -k (-mu)^{k-1}/(k+1)!
-            fact *= TA(k + 1);
-            dcoef = (k == 0) ? TA(0) : -TA(k) * pw / fact;
-            pw = (k == 0) ? TA(1) : pw * (-mu);
-            coef = pw / fact;
-            const TA *__restrict__ M = A.mom + (size_t)k * K * K;
-            TA gk = TA(0);
+        for (int i = 0; i < VPT; ++i) zs[i * VP * K + tid] = sum[i];
+    }
+    __syncthreads();
+    if constexpr (!f32) {
+        // the self block on the matrix instruction, as in k_combine
+        typedef double d4 __attribute__((ext_vector_type(4)));
+        constexpr int RT = (K + 15) / 16, CT = (VB + 15) / 16, KS = (K + 3) / 4;
+        const int lane = tid & (kWave - 1), n = lane & 15, gr = lane >> 4;
+        for (int u = tid / kWave; u < RT * CT; u += kCombThreads / kWave) {
+            const int rt = u % RT, vv = (u / RT) * 16 + n, vc = min(vv, VB - 1), row = min(rt * 16 + n, K - 1);
+            double x[2][KS], sum[2][4] = {};
 #pragma unroll
-            for (int a = 0; a < K; ++a) {
-                TA sx = TA(0), sw = TA(0);
-#pragma unroll
-                for (int b = 0; b < K; ++b) {
-                    sx += M[a * K + b] * xi[b];
-                    sw += M[a * K + b] * w[b];
-                }
-                acc[a] += A.self_scale * coef * sx;
-                gk += xi[a] * sw;
+            for (int s = 0; s < KS; ++s) {
+                const int b = 4 * s + gr, o = vc * K + min(b, K - 1);
+                const double xb = xs[o], wb = ws[o];
+                x[0][s] = b < K ? xb : 0.0;
+                x[1][s] = b < K ? wb : 0.0;
             }
-            gself += dcoef * gk;
+            const gptr<double> M = as_global<double>(A.mom) + (size_t)row * K;
+#pragma unroll 1
+            for (int k = 0; k < kNMom; ++k) {
+                d4 y[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    const double m = M[(size_t)k * K * K + min(4 * s + gr, K - 1)];
+                    y[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(m, x[0][s], y[0], 0, 0, 0);
+                    y[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(m, x[1][s], y[1], 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sum[0][r] += cf[0][k][vc] * y[0][r];
+                    sum[1][r] += cf[1][k][vc] * y[1][r];
+                }
+            }
+            // result r of a lane: row 4 r + gr, column n
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int ra = rt * 16 + 4 * r + gr;
+                if (vv < VB && ra < K) {
+                    sp[vv * K + ra] = sum[0][r];
+                    gp[vv * K + ra] = sum[1][r];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const int P = g.nx * g.ny;
+    if (live) {
+        const int l = l_of<L>(a);
+        const bool m0 = a == l * l + l;
+        TA gl = TA(1);
+#pragma unroll
+        for (int ll = 1; ll <= L; ++ll) gl = ll <= l ? gl * A.g_aniso : gl;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+            const int v = v0 + i * VP + q0, o = (i * VP + q0) * K;
+            TA acc = TA(0), st, gs;
+#pragma unroll
+            for (int t = 0; t < NZ; ++t) {  // back to the harmonic basis
+                const int j = tab.j[t][a];
+                if (j >= 0) acc = fmad(TA(tab.z[t][a]), zs[o + j], acc);
+            }
+            if constexpr (f32) {
+                T x[NJ], w[NJ], s32 = T(0), g32 = T(0);
+#pragma unroll
+                for (int t = 0; t < NJ; ++t) {
+                    const int b = tab.b[t][a];
+                    const T xb = xs[o + (b < 0 ? a : b)], wb = ws[o + (b < 0 ? a : b)];
+                    x[t] = b < 0 ? T(0) : xb;
+                    w[t] = b < 0 ? T(0) : wb;
+                }
+#pragma unroll 2
+                for (int k = 0; k < kNMom; ++k) {
+                    T rx = T(0), rw = T(0);
+#pragma unroll
+                    for (int t = 0; t < NJ; ++t) {
+                        const T m = ms[(k * NJ + t) * K + a];
+                        rx = t ? fmad(m, x[t], rx) : m * x[t];
+                        rw = t ? fmad(m, w[t], rw) : m * w[t];
+                    }
+                    s32 = fmad(cf[0][k][i * VP + q0], rx, s32);
+                    g32 = fmad(cf[1][k][i * VP + q0], rw, g32);
+                }
+                st = TA(s32);
+                gs = TA(xs[o + a] * g32);
+            } else {
+                st = sp[o + a];
+                gs = xs[o + a] * gp[o + a];
+            }
+            acc = (sgn * acc * na + A.self_scale * st) * A.dV;  // Lambda_q
+            gp[o + a] = gs;
+            const bool in = v < g.N;
+            const size_t e = (size_t)(in ? v : 0) * K + a;
+            sp[o + a] = A.aw_prev ? acc * gl * A.aw_prev[e] : TA(0);
+            if (!in) continue;
+            if (A.lam0 && m0) A.lam0[(size_t)v * (L + 1) + l] = acc;
+            TA xn = gl * TA(A.mus[v]) * acc;
+            if (m0 && v >= g.N - P) xn += A.cot[v - (g.N - P)] * A.coefE[l];
+            A.X[e] = T(sgn * xn * na);
         }
     }
-    A.gt[v] += A.self_scale * A.dV * gself;
-#pragma unroll
-    for (int a = 0; a < K; ++a) acc[a] *= A.dV;   // acc = Lambda_q(v)
-    const TA ms = TA(A.mus[v]);
-    if (A.aw_prev) {
-        TA gsv = TA(0), gl = TA(1);
-#pragma unroll
-        for (int l = 0; l <= L; ++l) {
-#pragma unroll
-            for (int m = -l; m <= l; ++m) gsv += acc[l * l + l + m] * gl * A.aw_prev[(size_t)v * K + l * l + l + m];
-            gl *= A.g_aniso;
+    __syncthreads();
+    if (tid < VB && v0 + tid < g.N) {
+        TA gt = TA(0), gs = TA(0);
+        for (int c = 0; c < K; ++c) {
+            gt += gp[tid * K + c];
+            gs += sp[tid * K + c];
         }
-        A.gs[v] += gsv;
-    }
-    if (A.lam0) {
-#pragma unroll
-        for (int l = 0; l <= L; ++l) A.lam0[(size_t)v * (L + 1) + l] = acc[l * l + l];
-    }
-    const int zk = v / (g.nx * g.ny);
-    const int pix = v - zk * g.nx * g.ny;
-    const bool bottom = (zk == g.nz - 1);
-    TA gl = TA(1);
-#pragma unroll
-    for (int l = 0; l <= L; ++l) {
-        const TA sgn = (l & 1) ? TA(-1) : TA(1);
-#pragma unroll
-        for (int m = -l; m <= l; ++m) {
-            const int a = l * l + l + m;
-            TA xn = gl * ms * acc[a];
-            if (m == 0 && bottom) xn += A.cot[pix] * A.coefE[l];
-            A.X[(size_t)v * K + a] = T(sgn * xn * A.nsc[a]);
-        }
-        gl *= A.g_aniso;
+        A.gt[v0 + tid] += A.self_scale * A.dV * gt;
+        if (A.aw_prev) A.gs[v0 + tid] += gs;
     }
 }
 
@@ -674,8 +733,10 @@ hipError_t launch_adj_prop(int L, const PropArgs<T> &A, int nc, const T *const *
 template <typename T, typename TA>
 hipError_t launch_adj_combine(int L, const AdjCombArgs<T, TA> &A, hipStream_t st)
 {
-    dim3 grid((A.g.N + kWave - 1) / kWave), block(kWave);
-    RTE_DISPATCH_L2(L, hipLaunchKernelGGL((k_adj_combine<T, TA, LL>), grid, block, 0, st, A));
+    RTE_DISPATCH_L2(L, {
+        constexpr int VB = CombShape<LL>::VB;
+        hipLaunchKernelGGL((k_adj_combine<T, TA, LL>), dim3((A.g.N + VB - 1) / VB), dim3(kCombThreads), 0, st, A);
+    });
     return hipGetLastError();
 }
 

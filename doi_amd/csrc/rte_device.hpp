@@ -386,36 +386,57 @@ __host__ __device__ constexpr bool self_couples(int a, int b)
     return sin_a == sin_b && ((am - bm) & 1) == 0 && ((la - lb) & 1) == 0;
 }
 
-// s += M[a][b] w[b] over the b that self_couples(a, b) keeps, and the same for
-// a second vector; unrolled at compile time, so the skipped entries cost nothing
-template <int a, int b, int K, typename T>
-__device__ __forceinline__ void self_term(T &s, const T *__restrict__ M, const T (&w)[K])
-{
-    if constexpr (self_couples(a, b)) s += M[a * K + b] * w[b];
-}
-template <int a, int K, typename T, int... bs>
-__device__ __forceinline__ T self_row(const T *__restrict__ M, const T (&w)[K], std::integer_sequence<int, bs...>)
-{
-    T s = T(0);
-    (self_term<a, bs, K>(s, M, w), ...);
-    return s;
-}
-// st[a] += coef * sum_b M[a][b] w[b] for every a (the kept entries)
-template <int K, typename T, int... as>
-__device__ __forceinline__ void self_apply(T (&st)[K], T coef, const T *__restrict__ M, const T (&w)[K],
-                                           std::integer_sequence<int, as...>)
-{
-    ((st[as] += coef * self_row<as, K>(M, w, std::make_integer_sequence<int, K>{})), ...);
-}
-// as self_apply, and gk += sum_a x[a] (M w)[a] (the mu-derivative term of the adjoint)
-template <int K, typename T, int... as>
-__device__ __forceinline__ void self_apply_adj(T (&st)[K], T &gk, T coef, const T *__restrict__ M,
-                                               const T (&x)[K], const T (&w)[K], std::integer_sequence<int, as...>)
-{
-    ((st[as] += coef * self_row<as, K>(M, x, std::make_integer_sequence<int, K>{}),
-      gk += x[as] * self_row<as, K>(M, w, std::make_integer_sequence<int, K>{})),
-     ...);
-}
+// The layout of the combine kernels (forward and adjoint): one thread per (voxel,
+// coefficient), VPT voxels each, VB voxels a block
+constexpr int kCombThreads = 256;
+
+template <int L>
+struct CombShape {
+    static constexpr int K = (L + 1) * (L + 1);
+    static constexpr int VP = kCombThreads / K < 64 ? kCombThreads / K : 64;  // voxels side by side
+    static constexpr int VPT = 2;                                            // voxels per thread
+    static constexpr int VB = VP * VPT;
+    static constexpr int coupled(int a)
+    {
+        int c = 0;
+        for (int b = 0; b < K; ++b) c += self_couples(a, b);
+        return c;
+    }
+    static constexpr int most()
+    {
+        int m = 0;
+        for (int a = 0; a < K; ++a) m = coupled(a) > m ? coupled(a) : m;
+        return m;
+    }
+    static constexpr int NJ = most();     // coupled coefficients of the self block
+    static constexpr int NZ = L / 2 + 1;  // z-power terms of a harmonic
+};
+
+// per coefficient: its coupled coefficients (ascending, padded with -1), and its
+// nonzero z-power terms (ascending, padded with -1)
+template <int L>
+struct CombTab {
+    using S = CombShape<L>;
+    short b[S::NJ][S::K], j[S::NZ][S::K];
+    double z[S::NZ][S::K];
+    constexpr CombTab() : b{}, j{}, z{}
+    {
+        for (int a = 0; a < S::K; ++a) {
+            for (int i = 0; i < S::NJ; ++i) b[i][a] = -1;
+            for (int i = 0; i < S::NZ; ++i) j[i][a] = -1;
+            int nb = 0, nz = 0;
+            for (int q = 0; q < S::K; ++q) {
+                if (self_couples(a, q)) b[nb++][a] = short(q);
+                if (kZPow<L>.m[a][q] != 0.0) {
+                    j[nz][a] = short(q);
+                    z[nz++][a] = kZPow<L>.m[a][q];
+                }
+            }
+        }
+    }
+};
+template <int L>
+static __constant__ constexpr CombTab<L> kCombTab{};
 
 // destination of a lane: brick blk, lane -> (di, dj, dk)
 template <typename T>

@@ -524,56 +524,6 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
 // once per tile instead of once per voxel.
 // grid = (ceil(N/VB), nsolve or ncomplex), block = kCombThreads.
 // ---------------------------------------------------------------------------
-constexpr int kCombThreads = 256;
-
-template <int L>
-struct CombShape {
-    static constexpr int K = (L + 1) * (L + 1);
-    static constexpr int VP = kCombThreads / K < 64 ? kCombThreads / K : 64;  // voxels side by side
-    static constexpr int VPT = 2;                                            // voxels per thread
-    static constexpr int VB = VP * VPT;
-    static constexpr int coupled(int a)
-    {
-        int c = 0;
-        for (int b = 0; b < K; ++b) c += self_couples(a, b);
-        return c;
-    }
-    static constexpr int most()
-    {
-        int m = 0;
-        for (int a = 0; a < K; ++a) m = coupled(a) > m ? coupled(a) : m;
-        return m;
-    }
-    static constexpr int NJ = most();     // coupled coefficients of the self block
-    static constexpr int NZ = L / 2 + 1;  // z-power terms of a harmonic
-};
-
-// per coefficient: its coupled coefficients (ascending, padded with -1), and its
-// nonzero z-power terms (ascending, padded with -1)
-template <int L>
-struct CombTab {
-    using S = CombShape<L>;
-    short b[S::NJ][S::K], j[S::NZ][S::K];
-    double z[S::NZ][S::K];
-    constexpr CombTab() : b{}, j{}, z{}
-    {
-        for (int a = 0; a < S::K; ++a) {
-            for (int i = 0; i < S::NJ; ++i) b[i][a] = -1;
-            for (int i = 0; i < S::NZ; ++i) j[i][a] = -1;
-            int nb = 0, nz = 0;
-            for (int q = 0; q < S::K; ++q) {
-                if (self_couples(a, q)) b[nb++][a] = short(q);
-                if (kZPow<L>.m[a][q] != 0.0) {
-                    j[nz][a] = short(q);
-                    z[nz++][a] = kZPow<L>.m[a][q];
-                }
-            }
-        }
-    }
-};
-template <int L>
-__constant__ constexpr CombTab<L> kCombTab{};
-
 template <typename T, typename TA, int L, int NH>
 __global__ __launch_bounds__(kCombThreads) void k_combine(CombArgs<T, TA> A, const SolveDev<T, TA> *__restrict__ sv)
 {

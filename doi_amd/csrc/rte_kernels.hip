@@ -42,7 +42,8 @@ __global__ void k_fill(T *__restrict__ p, size_t n, T v)
 //   Group z holds the NR solves sv[z*NR .. z*NR+NR-1], which share one medium
 //   (same path table and mu_t): the pair direction, its z-power values and kf
 //   are computed once and applied to every right-hand side.
-// PATH 0: kf from the per-medium table; PATH 1: marched per pair.
+// PATH 0: kf from the per-medium table; PATH 1: marched per pair; PATH 2: marched with
+// the map of mu_t in LDS.
 // ---------------------------------------------------------------------------
 constexpr int kPropWaves = 4;
 template <typename T, typename TA, int L, int PATH, int NR, bool CPLX = false, bool SEP = false>
@@ -58,8 +59,14 @@ __global__ __launch_bounds__(kWave * kPropWaves) void k_prop(PropArgs<T> A, cons
     const GridDev<T> &g = A.g;
     const int lane = threadIdx.x % kWave, blk = blockIdx.x * kPropWaves + threadIdx.x / kWave;
     const int chunk = blockIdx.y;
-    if (blk >= g.nblk) return;  // the last workgroup's waves past the last brick (no barriers follow)
     const SolveDev<T, TA> *__restrict__ grp = sv + (size_t)blockIdx.z * NR;
+    extern __shared__ __align__(16) unsigned char prop_lds[];
+    if constexpr (PATH == 2) {
+        T *sm = reinterpret_cast<T *>(prop_lds);
+        for (int i = threadIdx.x; i < g.N; i += kWave * kPropWaves) sm[i] = grp[0].mut[i];
+        __syncthreads();
+    }
+    if (blk >= g.nblk) return;  // the last workgroup's waves past the last brick (no barriers follow)
     int di, dj, dk;
     lane_dest(g, blk, lane, di, dj, dk);
     const bool valid = di < g.nx && dj < g.ny && dk < g.nz;
@@ -139,7 +146,13 @@ __global__ __launch_bounds__(kWave * kPropWaves) void k_prop(PropArgs<T> A, cons
             const int ix = cdi - si, iy = cdj - sj, iz = cdk - sk;
             const bool use = valid && !self && (r2 < A.thr2);
             const T r = sqrt(self ? T(1) : r2);
-            const T tau = use ? march_tau<T>(mut, s, ix, iy, iz, g.nx, nxy, r) : T(0);
+            T tau = T(0);
+            if (use) {
+                if constexpr (PATH == 2)
+                    tau = march_tau<T>((const __attribute__((address_space(3))) T *)prop_lds, s, ix, iy, iz, g.nx, nxy, r);
+                else
+                    tau = march_tau<T>(mut, s, ix, iy, iz, g.nx, nxy, r);
+            }
             kfs[0] = use ? dev_exp<T>(-tau) / r2 : T(0);
             r2 = self ? T(1) : r2;
         }
@@ -1217,6 +1230,11 @@ hipError_t launch_to_zpow(int L, int N, const SolveDev<T, TA> *sv, int nsolve, h
     return hipGetLastError();
 }
 
+// The marched FP32 propagation up to L = 5 reads mu_t from LDS up to this size of the map,
+// which leaves 5 workgroups a CU (ms a term, memory / LDS: 16^3 L = 5 0.332 / 0.292, 20^3
+// L = 3 1.27 / 1.11, 22^3 L = 5 3.11 / 3.30, 24^3 L = 3 4.08 / 4.28)
+constexpr size_t kMarchLds = 32 << 10;
+
 template <typename T, typename TA>
 hipError_t launch_prop(int L, int path, int nr, const PropArgs<T> &A, const SolveDev<T, TA> *sv, int ngroups,
                        hipStream_t st)
@@ -1235,6 +1253,13 @@ hipError_t launch_prop(int L, int path, int nr, const PropArgs<T> &A, const Solv
     if (e != hipSuccess) return e;
     RTE_DISPATCH_L(L, {
         if (path == 1) {
+            if constexpr (sizeof(T) == 4 && LL <= 5) {
+                const size_t map = (size_t)A.g.N * sizeof(T);
+                if (map <= kMarchLds) {
+                    hipLaunchKernelGGL((k_prop<T, TA, LL, 2, 1>), grid, block, map, st, A, sv);
+                    break;
+                }
+            }
             hipLaunchKernelGGL((k_prop<T, TA, LL, 1, 1>), grid, block, 0, st, A, sv);
         } else if constexpr (multi) {
             switch (nr) {

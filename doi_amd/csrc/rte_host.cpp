@@ -89,39 +89,6 @@ struct DevBuf {
     T *as() const { return static_cast<T *>(p); }
 };
 
-// Pinned host memory that kernels write their results to (kept, grown as needed): a small
-// copy back costs a launch of the runtime's copy kernel and its staging, ~10 us each; with
-// the descriptors' uploads only when they change, a 8^3 solve of 8 terms 610 -> 458 us
-struct PinBuf {
-    void *p = nullptr;
-    size_t bytes = 0;
-    PinBuf() = default;
-    PinBuf(const PinBuf &) = delete;
-    PinBuf &operator=(const PinBuf &) = delete;
-    ~PinBuf() { release(); }
-    void release()
-    {
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-        bytes = 0;
-    }
-    hipError_t alloc(size_t n)
-    {
-        if (n <= bytes && p) return hipSuccess;
-        release();
-        const hipError_t e = hipHostMalloc(&p, n ? n : 16, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
-            return e;
-        }
-        bytes = n;
-        return hipSuccess;
-    }
-    template <typename T>
-    T *as() const { return static_cast<T *>(p); }
-};
-
 // ---------------------------------------------------------------------------
 // host-side math: SH recurrence constants, exitance weights, self-block grid
 // ---------------------------------------------------------------------------
@@ -357,9 +324,9 @@ struct rte_ctx {
     std::list<ZTab> ztabs;  // Z tables of the matrix-core propagation, last used first
     std::mutex ztabs_mu;    // (a server's thread uses them too)
     // solve workspace (grow-only)
-    DevBuf ws_W, ws_Wp, ws_part, ws_pix, ws_sv, ws_beams;
+    DevBuf ws_W, ws_Wp, ws_part, ws_pix, ws_sv, ws_beams, ws_red;
     std::set<rte_medium *> media;  // live media of this context
-    PinBuf pin_red, pin_img;  // sums of a term, images of a batch
+    std::vector<char> host_red;
 };
 
 struct rte_medium {
@@ -1018,7 +985,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
     HIP_TRY(ctx->ws_Wp.alloc(sh.wp * sizeof(T) * ns));
     HIP_TRY(ctx->ws_part.alloc(szPart * sizeof(T) * ns));
     HIP_TRY(ctx->ws_pix.alloc((size_t)kPixBufs * P * sizeof(TA) * ns));
-    HIP_TRY(ctx->pin_red.alloc((size_t)2 * sizeof(TA) * ns));
+    HIP_TRY(ctx->ws_red.alloc((size_t)2 * sizeof(TA) * ns));
     HIP_TRY(ctx->ws_sv.alloc(sizeof(SolveDev<T, TA>) * ns * 2));
     HIP_TRY(ctx->ws_beams.alloc(sizeof(BeamDev) * nb));
 
@@ -1039,7 +1006,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
             s.mus = sizeof(T) == 4 ? (const T *)m->mus_f.p : (const T *)m->mus_d.p;
             s.g = T(m->g);
             set_pixels(s, ctx->ws_pix.as<TA>() + (size_t)kPixBufs * P * q, P);
-            s.red = ctx->pin_red.as<TA>() + 2 * q;
+            s.red = ctx->ws_red.as<TA>() + 2 * q;
             s.mode = 1;
             s.kim = kim ? T(kim[i]) : T(0);
         }
@@ -1123,7 +1090,9 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
         HIP_TRY(launch_bottom<T, TA>(P, svd, ns, st));
         tm.done();
     }
-    const volatile TA *red = ctx->pin_red.as<TA>();  // written by launch_bottom
+    ctx->host_red.resize(sizeof(TA) * 2 * ns);
+    TA *red = reinterpret_cast<TA *>(ctx->host_red.data());
+    HIP_TRY(hipMemcpyAsync(red, ctx->ws_red.p, sizeof(TA) * 2 * ns, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     for (int i = 0; i < nb; ++i) {
         HostSolve &h = hs[i];
@@ -1165,7 +1134,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
     }
 
     std::vector<int> act;
-    std::vector<SolveDev<T, TA>> svact, svgrp, svup;  // svup: what svd holds
+    std::vector<SolveDev<T, TA>> svact, svgrp;
     SolveDev<T, TA> *svd_grp = svd + nb;
     for (;;) {
         act.clear();
@@ -1179,14 +1148,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
                 svact[j * hv + hh].mode = hs[act[j]].state;
             }
         const int na = (int)act.size();
-        // the descriptors go up when they differ from the last term's (a solve has ended)
-        const size_t actb = sizeof(SolveDev<T, TA>) * na * hv;
-        const bool fresh = svup.size() != svact.size() || std::memcmp(svup.data(), svact.data(), actb) != 0;
-        if (fresh) {
-            HIP_TRY(hipMemcpyAsync(svd, svact.data(), actb, hipMemcpyHostToDevice, st));
-            svup.resize(svact.size());
-            std::memcpy((void *)svup.data(), svact.data(), actb);
-        }
+        HIP_TRY(hipMemcpyAsync(svd, svact.data(), sizeof(SolveDev<T, TA>) * na * hv, hipMemcpyHostToDevice, st));
         if (kim) {
             LaunchTimer tm(ctx, 0);
             HIP_TRY(launch_prop_c<T, TA>(L, path, pa, svd, na, st));
@@ -1201,9 +1163,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
                                  [&](int a, int b) { return svact[a].ktab < svact[b].ktab; });
                 svgrp.clear();
                 for (int j : order) svgrp.push_back(svact[j]);
-                if (fresh)
-                    HIP_TRY(hipMemcpyAsync(svd_grp, svgrp.data(), sizeof(SolveDev<T, TA>) * na, hipMemcpyHostToDevice,
-                                           st));
+                HIP_TRY(hipMemcpyAsync(svd_grp, svgrp.data(), sizeof(SolveDev<T, TA>) * na, hipMemcpyHostToDevice, st));
                 {
                     LaunchTimer tm(ctx, 2);
                     HIP_TRY(launch_to_pieces<TA>(L, g, svd_grp, na, st));
@@ -1262,9 +1222,8 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
             }
             const int sep_off = (int)svgrp.size();
             for (int q : sep) svgrp.push_back(svact[q]);
-            if (fresh)
-                HIP_TRY(hipMemcpyAsync(svd_grp, svgrp.data(), sizeof(SolveDev<T, TA>) * svgrp.size(),
-                                       hipMemcpyHostToDevice, st));
+            HIP_TRY(hipMemcpyAsync(svd_grp, svgrp.data(), sizeof(SolveDev<T, TA>) * svgrp.size(),
+                                   hipMemcpyHostToDevice, st));
             for (auto &ln : launches) {
                 const int k = ln.first, ng = (int)by_size[k].size() / k;
                 LaunchTimer tm(ctx, 0, k);
@@ -1286,15 +1245,17 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
             HIP_TRY(launch_bottom<T, TA>(P, svd, na * hv, st));
             tm.done();
         }
+        std::vector<TA> r(2 * ns);
+        HIP_TRY(hipMemcpyAsync(r.data(), ctx->ws_red.p, sizeof(TA) * 2 * ns, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
         const double now_ms =
             std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
         for (int j = 0; j < na; ++j) {
             HostSolve &h = hs[act[j]];
             const int q = act[j] * hv;
-            const double dT = (double)red[2 * q];
-            const double sumW = (double)red[2 * q + 1] + (hv == 2 ? (double)red[2 * q + 3] : 0.0);
-            const double dTi = hv == 2 ? (double)red[2 * q + 2] : 0.0;
+            const double dT = (double)r[2 * q];
+            const double sumW = (double)r[2 * q + 1] + (hv == 2 ? (double)r[2 * q + 3] : 0.0);
+            const double dTi = hv == 2 ? (double)r[2 * q + 2] : 0.0;
             lat[act[j]] = now_ms;
             advance_series(h, dT, sumW, p->stop_rule, p->tol, max_terms, dTi);
         }
@@ -1302,15 +1263,17 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
     }
     HIP_TRY(hipEventRecord(ctx->ev1, st));
     // gather exitance images (a complex solve: real plane, then imaginary plane)
-    const int planes = reflectance ? 2 : 1;
-    HIP_TRY(ctx->pin_img.alloc((size_t)planes * ns * P * sizeof(TA)));
-    TA *img = ctx->pin_img.as<TA>();
-    HIP_TRY(launch_pixels<TA>(P, kPixBufs * P, sv[0].E, img, ns, st));
-    if (reflectance) HIP_TRY(launch_pixels<TA>(P, kPixBufs * P, sv[0].R, img + (size_t)ns * P, ns, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    for (size_t q = 0; q < (size_t)ns * P; ++q) exitance[q] = (double)img[q];
-    if (reflectance)
-        for (size_t q = 0; q < (size_t)ns * P; ++q) reflectance[q] = (double)img[(size_t)ns * P + q];
+    std::vector<TA> img((size_t)P);
+    for (int q0 = 0; q0 < ns; ++q0) {
+        HIP_TRY(hipMemcpyAsync(img.data(), sv[q0].E, sizeof(TA) * P, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        for (int q = 0; q < P; ++q) exitance[(size_t)q0 * P + q] = (double)img[q];
+        if (reflectance) {
+            HIP_TRY(hipMemcpyAsync(img.data(), sv[q0].R, sizeof(TA) * P, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+            for (int q = 0; q < P; ++q) reflectance[(size_t)q0 * P + q] = (double)img[q];
+        }
+    }
     if (want_cplx) {
         // the reference's complex basis and layout, converted on the device
         DevBuf dC;

@@ -169,6 +169,9 @@ hipError_t launch_combine_c(int L, const CombArgs<T, TA> &A, const SolveDev<T, T
                             hipStream_t st);
 template <typename T, typename TA>
 hipError_t launch_bottom(int P, const SolveDev<T, TA> *sv, int nsolve, hipStream_t st);
+// the images of nsolve solves whose pixel buffers lie stride elements apart, one after another
+template <typename TA>
+hipError_t launch_pixels(int P, int stride, const TA *pix, TA *out, int nsolve, hipStream_t st);
 template <typename T, typename TA>
 hipError_t launch_source(int L, const GridDev<T> &g, double dx, double dy, double dz, double xmin,
                          double ymin, const Scales &sc, const BeamDev *beams, const SolveDev<T, TA> *sv,

@@ -859,6 +859,14 @@ __global__ __launch_bounds__(256) void k_bottom(int P, const SolveDev<T, TA> *__
     }
 }
 
+// grid = (ceil(P/256), nsolve), block = 256
+template <typename TA>
+__global__ __launch_bounds__(256) void k_pixels(int P, int stride, const TA *__restrict__ pix, TA *__restrict__ out)
+{
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < P) out[(size_t)blockIdx.y * P + p] = pix[(size_t)blockIdx.y * stride + p];
+}
+
 // ---------------------------------------------------------------------------
 // First-scatter source s0 and ballistic image (column products, FP64):
 //   s0_l0(i,j,k) = fact g^l sqrt((2l+1)/4pi) (mu_s/mu_t) T(k) (1 - e^{-mu_t dz}) / dV
@@ -1402,6 +1410,13 @@ hipError_t launch_bottom(int P, const SolveDev<T, TA> *sv, int nsolve, hipStream
     return hipGetLastError();
 }
 
+template <typename TA>
+hipError_t launch_pixels(int P, int stride, const TA *pix, TA *out, int nsolve, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_pixels<TA>), dim3((P + 255) / 256, nsolve), dim3(256), 0, st, P, stride, pix, out);
+    return hipGetLastError();
+}
+
 template <typename T, typename TA>
 hipError_t launch_source(int L, const GridDev<T> &g, double dx, double dy, double dz, double xmin,
                          double ymin, const Scales &sc, const BeamDev *beams, const SolveDev<T, TA> *sv,
@@ -1539,6 +1554,8 @@ template hipError_t launch_combine<double, double>(int, const CombArgs<double, d
                                                    const SolveDev<double, double> *, int, hipStream_t);
 template hipError_t launch_combine<float, float>(int, const CombArgs<float, float> &,
                                                  const SolveDev<float, float> *, int, hipStream_t);
+template hipError_t launch_pixels<float>(int, int, const float *, float *, int, hipStream_t);
+template hipError_t launch_pixels<double>(int, int, const double *, double *, int, hipStream_t);
 template hipError_t launch_bottom<float, double>(int, const SolveDev<float, double> *, int,
                                                  hipStream_t);
 template hipError_t launch_bottom<double, double>(int, const SolveDev<double, double> *, int,

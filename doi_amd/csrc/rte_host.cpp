@@ -110,7 +110,7 @@ struct TablePool {
     ~TablePool();
     void put(DevBuf &b)
     {
-        {
+        try {
             std::lock_guard<std::mutex> lk(mu);
             if (b.p && bytes + b.bytes <= kTablesKeep) {
                 kept.emplace_back(b.p, b.bytes);
@@ -118,6 +118,7 @@ struct TablePool {
                 b.p = nullptr;
                 b.bytes = 0;
             }
+        } catch (const std::bad_alloc &) {  // no room for the list: freed as before
         }
         b.release();
     }
@@ -3416,6 +3417,7 @@ extern "C" int rte_server_create(rte_ctx *ctx, const rte_server_opts *opts, rte_
     if (S->opts.hbm_budget <= 0) {
         size_t fr = 0, tot = 0;
         HIP_TRY(hipSetDevice(ctx->device));
+        give_back_tables();  // kept memory counts as free
         HIP_TRY(hipMemGetInfo(&fr, &tot));
         S->opts.hbm_budget = (long long)(0.8 * (double)fr);
     }

@@ -56,7 +56,7 @@ struct SolveDev {
     T *Wp;             // [N][K] the same in the propagation's z-power basis, written by each launch
     T *part;           // [nchunk][N][K] partial pair sums
     const T *ktab;     // [N][npad] e^{-tau}/r^2 per (source, destination slot), cached mode
-    const unsigned char *kexp;  // [slab][npad] exponents of the path table (rte_mfma.hip), if it is used there
+    const unsigned char *kexp;  // [slab + 1][npad] exponents of the path table (rte_mfma.hip), if it is used there
     const T *mut;      // [N] mu_t
     const T *mus;      // [N] mu_s
     T g;               // anisotropy

@@ -169,7 +169,9 @@ __global__ __launch_bounds__(kWave) void k_to_pieces(GridDev<float> g, const Sol
 // ---------------------------------------------------------------------------
 // The exponents of the path table: byte [slab][slot] is the biased exponent of the
 // largest kf of the slab's (up to 16) sources for that destination.  T is scaled with it.
-// grid = (ceil(npad / 1024), slabs), block = 256: 4 slots per thread.
+// After the last slab the exponents of the slab of zeros, all 127: the entries read beside
+// it are a neighbour's, of any size, and have to stay finite for T to be 0.
+// grid = (ceil(npad / 1024), slabs + 1), block = 256: 4 slots per thread.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_kexp(GridDev<float> g, const float *__restrict__ ktab,
                                               unsigned *__restrict__ kexp)
@@ -177,6 +179,10 @@ __global__ __launch_bounds__(256) void k_kexp(GridDev<float> g, const float *__r
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= g.npad / 4) return;
     const int slab = blockIdx.y, z = slab % g.nz, b = slab / g.nz;
+    if (slab == g.bx * g.by * g.nz) {
+        kexp[(size_t)slab * (g.npad / 4) + q] = 0x7f7f7f7fu;
+        return;
+    }
     const int x0 = (b % g.bx) * kBrick, y0 = (b / g.bx) * kBrick;
     const f4 *__restrict__ row = reinterpret_cast<const f4 *>(ktab) + q;
     f4 m = {0.f, 0.f, 0.f, 0.f};
@@ -471,7 +477,7 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void k_prop_mfma(MfmaArgs A, const
             const GLBP unsigned char *w = *(const GLBP unsigned char * const LDSP *)(lds + D::PTR + cc * 16 + 8);
             const GLBP unsigned char *ke = *(const GLBP unsigned char * const LDSP *)(lds + D::PTR + 256 + cc * 8);
             sn = *(const GLBP float *)(w + ((unsigned long long)(unsigned)nslab + 1) * 16 * M::WB + (unsigned)sl * 4ull);
-            en = *(const GLBP u4 *)(ke + (unsigned)(sl < nslab ? sl : 0) * (unsigned long long)g.npad + (unsigned)slot);
+            en = *(const GLBP u4 *)(ke + (unsigned)sl * (unsigned long long)g.npad + (unsigned)slot);
         };
         {
             const KPtr k = kptr(at, z);
@@ -745,11 +751,11 @@ double mfma_translations(const GridDev<float> &g, int nr, int *ntx, int *ntz)
     return best;
 }
 
-size_t kexp_bytes(const GridDev<float> &g) { return (size_t)g.bx * g.by * g.nz * g.npad; }
+size_t kexp_bytes(const GridDev<float> &g) { return ((size_t)g.bx * g.by * g.nz + 1) * g.npad; }
 
 hipError_t launch_kexp(const GridDev<float> &g, const float *ktab, unsigned char *kexp, hipStream_t st)
 {
-    const dim3 grid((g.npad + 1023) / 1024, g.bx * g.by * g.nz);
+    const dim3 grid((g.npad + 1023) / 1024, g.bx * g.by * g.nz + 1);
     hipLaunchKernelGGL(k_kexp, grid, dim3(256), 0, st, g, ktab, reinterpret_cast<unsigned *>(kexp));
     return hipGetLastError();
 }

@@ -55,11 +55,13 @@ struct MLay {
 
 constexpr float kZScale = 1024.f;                     // Z pieces hold 2^10 Z
 
-// split x = h + l: h the leading 11 bits, l rounded to FP16
+// split x = h + l, both rounded to nearest: |l| <= 2^-12 |x|, of either sign, so that the l l
+// products that are left out are below 2^-24 and do not add up.  Error of A W against FP64,
+// rms relative to k_prop's, mean over 24 media of 32^3: first term of a pencil beam 1.01
+// (with h cut off, every l of x's sign, 1.47), the next four terms 0.3.
 __device__ __forceinline__ void split2(float x, _Float16 &h, _Float16 &l)
 {
-    const float hf = __uint_as_float(__float_as_uint(x) & 0xffffe000u);
-    h = (_Float16)hf;
+    h = (_Float16)x;
     l = (_Float16)(x - (float)h);
 }
 

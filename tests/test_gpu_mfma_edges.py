@@ -1,9 +1,11 @@
 """The matrix-core propagation where a column of its products has no source in a tile, on
 grids of small voxels: the path-table entries read there (up to 1/pitch^2) belong to other
 sources than the exponents that scale them, which are 0 beyond the coupling threshold and
-where the path integral across the grid underflows.
+where the path integral across the grid underflows.  And the bits that its operands keep.
 
-Tolerance (max |difference| / max |reference|): the mixed operators' 1e-5.
+Tolerances: max |difference| / max |reference|, the mixed operators' 1e-5; a pencil beam's
+first term, whose sums are short, root mean square 4 x 2^-24 (a rounding to 24 bits of the
+table, the harmonics, the coefficients and the weighted projections).
 """
 import numpy as np
 import pytest
@@ -26,3 +28,13 @@ def test_columns_without_a_source(ctx, L, shape, thr, mus):
     assert np.isfinite(got).all() and np.isfinite(got32).all()
     assert rel_max(got, ref) < 1e-5
     assert rel_max(got32, ref) < 1e-5
+
+
+def test_short_sums_keep_24_bits(ctx):
+    shape, L, g = (32, 32, 32), 5, 0.8
+    bounds, N = bounds_for(shape), 32 ** 3
+    ma, ms = np.full(N, 0.25), np.full(N, 4.75)
+    W = ctx.source(shape, bounds, ma, ms, g, (0.05, 0.05, 0.1, 1.0), L)[0]
+    print("short sums", flush=True)
+    ref, got = (ctx.propagate(shape, bounds, ma, ms, g, W, L, precision=p) for p in (rte.PREC_FP64, rte.PREC_MIXED))
+    assert np.sqrt(np.mean((got - ref) ** 2) / np.mean(ref ** 2)) < 4 * 2.0 ** -24

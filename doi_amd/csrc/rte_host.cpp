@@ -442,6 +442,22 @@ struct rte_ctx {
     PinBuf pin_red, pin_img;  // sums of a term, images of a batch
 };
 
+// What the choice of the propagation looks at in a medium
+struct OptRange {
+    double mut_max = 0, mus_min = 0, mus_max = 0;
+};
+
+static OptRange opt_range(const double *mua, const double *mus, size_t N)
+{
+    OptRange r{0.0, N ? mus[0] : 0.0, 0.0};
+    for (size_t v = 0; v < N; ++v) {
+        r.mut_max = std::max(r.mut_max, mua[v] + mus[v]);
+        r.mus_min = std::min(r.mus_min, mus[v]);
+        r.mus_max = std::max(r.mus_max, mus[v]);
+    }
+    return r;
+}
+
 struct rte_medium {
     rte_ctx *ctx = nullptr;
     rte_grid grid{};
@@ -455,6 +471,7 @@ struct rte_medium {
     double ktab_f_thr = -1, ktab_d_thr = -1;
     DevBuf kexp;  // exponents of ktab_f, if kexp_ok
     bool kexp_ok = false;
+    OptRange range;
 };
 
 static int set_device(rte_ctx *ctx)
@@ -682,6 +699,7 @@ extern "C" int rte_medium_create(rte_ctx *ctx, const rte_grid *grid, const rte_o
     const size_t N = (size_t)m->N;
     m->mua_h.assign(optics->mu_a, optics->mu_a + N);
     m->mus_h.assign(optics->mu_s, optics->mu_s + N);
+    m->range = opt_range(optics->mu_a, optics->mu_s, N);
     std::vector<float> mt_f(N), ms_f(N);
     std::vector<double> mt_d(N);
     for (size_t v = 0; v < N; ++v) {
@@ -837,20 +855,40 @@ static double mfma_chunks(const GridDev<float> &g, int K, int *nchunk)
     return best;
 }
 
+// Whether the matrix cores' products keep a medium's small values.  A slab's 16 sources
+// share their scales (the largest |W|, the largest table entry of the destination), so a
+// contribution has ~2^-35 of (largest entry) x (largest W) as its error.  The slab's
+// strongest source contributes its W times its own entry: the error stays below FP32's
+// where a slab's entries differ by less than 600 (cubes of optical thickness 1, whose nearest
+// and farthest source are 1 and at most sqrt 19 voxels away: 19 e^3.4).  With a coupling
+// threshold that source may be beyond it: then a threshold of two bricks and mu_s within 64
+// are asked for too.  Error of A W against FP64 at 32^3, a pencil beam's first terms, worst
+// voxel relative to its own value, matrix cores (k_prop): thickness 1 1.7e-5 (1.9e-5), 2 1.0e-4
+// (4e-5), 3 2.9e-3 (5.5e-5), 6 1.0 (5e-5); thickness 0.1, threshold 2.5 voxels, mu_s within
+// 10^7 1.2e-2 (3e-5); all of thickness up to 1, thresholds from 8 voxels, mu_s within 64:
+// 1.0e-4 (5e-5).
+static bool even_medium(const rte_grid &gr, const OptRange &r, double thr)
+{
+    const double dx = (gr.xmax - gr.xmin) / gr.nx, dy = (gr.ymax - gr.ymin) / gr.ny, dz = (gr.zmax - gr.zmin) / gr.nz;
+    const double near = std::min(std::min(dx, dy), dz), far = std::sqrt(9.0 * (dx * dx + dy * dy) + dz * dz);
+    if (!(far * far / (near * near) * std::exp(r.mut_max * (far - near)) <= 600.0)) return false;
+    return thr <= 0.0 || (thr >= 2 * kBrick * std::max(dx, dy) && r.mus_max <= 64.0 * r.mus_min);
+}
+
 // Whether the FP32 cached propagation of a grid runs on the matrix cores (rte_mfma.hip):
 // L = 4 and 5, where a solve alone is to take at most 0.95 of k_prop's time there (2.34
 // and 2.94 ps a pair), which is where no group of solves measured slower.  It depends on
-// the grid and order only, so that a solve takes the same kernel, and has the same bits,
-// alone and in any batch.
-static bool use_mfma(int L, const GridDev<float> &g)
+// the grid, the order and the solve's medium (even) only, so that a solve takes the same
+// kernel, and has the same bits, alone and in any batch.
+static bool use_mfma(int L, const GridDev<float> &g, bool even)
 {
-    if (L != 4 && L != 5) return false;
+    if (!even || (L != 4 && L != 5)) return false;
     int nch = 1;
     return mfma_chunks(g, (L + 1) * (L + 1), &nch) < 0.95 * (L == 4 ? 2.34e-6 : 2.94e-6) * g.N * (double)g.N;
 }
 
 // The chunks of a propagation and the size of its input copy Wp (in T); depends on
-// the grid, order and path only, so that a solve's partial sums, and its bits, are the
+// the grid, order, path and medium only, so that a solve's partial sums, and its bits, are the
 // same alone and in any batch.
 struct PropShape {
     bool mfma = false;
@@ -859,12 +897,12 @@ struct PropShape {
 };
 
 template <typename T>
-static PropShape prop_shape(const GridDev<T> &g, int L, int path, bool cplx)
+static PropShape prop_shape(const GridDev<T> &g, int L, int path, bool cplx, bool even)
 {
     PropShape s;
     const int K = (L + 1) * (L + 1);
     if constexpr (sizeof(T) == 4) {
-        if (path == RTE_PATH_CACHED && !cplx && use_mfma(L, g)) {
+        if (path == RTE_PATH_CACHED && !cplx && use_mfma(L, g, even)) {
             s.mfma = true;
             mfma_chunks(g, K, &s.nch);
             s.wp = mfma_wp_bytes(L, g) / sizeof(T);
@@ -1043,6 +1081,7 @@ struct RefSrc {
     double *cplx_field = nullptr; // host, [N][K] complex: the final field in the reference's layout
 };
 
+// (the media of a batch are all even, or none is: solve_images)
 template <typename T, typename TA>
 static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
                      const rte_params *p, double *exitance, rte_stats *stats, const RefSrc<TA> *rs = nullptr,
@@ -1084,7 +1123,7 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
         for (int i = 0; i < nb; ++i)
             if ((rc = ensure_ktab<T>(media[i], thr))) return rc;
 
-    const PropShape sh = prop_shape<T>(g, L, path, kim != nullptr);
+    const PropShape sh = prop_shape<T>(g, L, path, kim != nullptr, even_medium(grid, media[0]->range, thr));
     const int nch = sh.nch;
     PropArgs<T> pa;
     std::shared_ptr<DevBuf> zt;
@@ -1448,6 +1487,19 @@ static int check_params(const rte_params *p)
     return RTE_OK;
 }
 
+static int solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
+                        const rte_params *params, double *exitance, double *reflectance, rte_stats *stats)
+{
+    switch (params->precision) {
+    case RTE_PREC_FP64:
+        return run_batch<double, double>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
+    case RTE_PREC_MIXED:
+        return run_batch<float, double>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
+    default:
+        return run_batch<float, float>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
+    }
+}
+
 extern "C" int rte_solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
                                 const rte_params *params, double *exitance, double *reflectance, rte_stats *stats)
 {
@@ -1466,14 +1518,47 @@ extern "C" int rte_solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, 
             return fail(RTE_E_ARG, "beam %d invalid", i);
     }
     if ((rc = set_device(ctx))) return rc;
-    switch (params->precision) {
-    case RTE_PREC_FP64:
-        return run_batch<double, double>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
-    case RTE_PREC_MIXED:
-        return run_batch<float, double>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
-    default:
-        return run_batch<float, float>(ctx, nb, media, beams, params, exitance, stats, nullptr, reflectance);
+    // solves that the matrix cores take and solves that they do not are batches of their own
+    const GridDev<float> g = make_grid<float>(media[0]->grid);
+    std::vector<int> on, off;
+    if (params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED && use_mfma(params->L, g, true))
+        for (int i = 0; i < nb; ++i)
+            (even_medium(media[i]->grid, media[i]->range, params->prop_thresh) ? on : off).push_back(i);
+    if (on.empty() || off.empty()) return solve_images(ctx, nb, media, beams, params, exitance, reflectance, stats);
+    const size_t P = (size_t)media[0]->grid.nx * media[0]->grid.ny;
+    double gpu_ms = 0.0;
+    std::vector<rte_stats> stat(nb);
+    const auto t0 = std::chrono::steady_clock::now();
+    for (const std::vector<int> *part : {&on, &off}) {
+        const int n = (int)part->size();
+        const double before =
+            std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        std::vector<rte_medium *> m(n);
+        std::vector<rte_beam> b(n);
+        std::vector<rte_stats> s(n);
+        std::vector<double> img(P * n), refl(reflectance ? P * n : 0);
+        for (int j = 0; j < n; ++j) {
+            m[j] = media[(*part)[j]];
+            b[j] = beams[(*part)[j]];
+        }
+        if ((rc = solve_images(ctx, n, m.data(), b.data(), params, img.data(), reflectance ? refl.data() : nullptr,
+                               s.data())))
+            return rc;
+        gpu_ms += s[0].gpu_ms;
+        for (int j = 0; j < n; ++j) {
+            const int i = (*part)[j];
+            std::copy_n(&img[P * j], P, exitance + P * i);
+            if (reflectance) std::copy_n(&refl[P * j], P, reflectance + P * i);
+            stat[i] = s[j];
+            stat[i].latency_ms += before;
+        }
     }
+    if (stats)
+        for (int i = 0; i < nb; ++i) {
+            stats[i] = stat[i];
+            stats[i].gpu_ms = gpu_ms;
+        }
+    return RTE_OK;
 }
 
 extern "C" int rte_solve_media(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
@@ -1704,6 +1789,15 @@ extern "C" int rte_solve(rte_ctx *ctx, const rte_grid *grid, const rte_optics *o
     return rc;
 }
 
+extern "C" int rte_on_matrix_cores(const rte_medium *m, const rte_params *params)
+{
+    if (!m) return fail(RTE_E_ARG, "rte_on_matrix_cores: NULL medium");
+    int rc;
+    if ((rc = check_params(params))) return rc;
+    return params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
+           use_mfma(params->L, make_grid<float>(m->grid), even_medium(m->grid, m->range, params->prop_thresh));
+}
+
 extern "C" long long rte_solve_footprint(const rte_grid *grid, const rte_params *params, int path_mode)
 {
     if (!grid || !params || params->L < 0 || params->L > RTE_MAX_L) return -1;
@@ -1713,9 +1807,9 @@ extern "C" long long rte_solve_footprint(const rte_grid *grid, const rte_params 
     const long long N = g.N;
     // the larger of the shapes that solves of this grid and order take; the 1/64 of a path table
     // that the matrix cores' exponents take, and the Z table that a grid's solves share, not counted
-    PropShape sh = prop_shape<float>(g, params->L, RTE_PATH_MARCH, false);
+    PropShape sh = prop_shape<float>(g, params->L, RTE_PATH_MARCH, false, true);
     if (params->precision != RTE_PREC_FP64) {
-        const PropShape m = prop_shape<float>(g, params->L, RTE_PATH_CACHED, false);
+        const PropShape m = prop_shape<float>(g, params->L, RTE_PATH_CACHED, false, true);
         sh.nch = std::max(sh.nch, m.nch);
         sh.wp = std::max(sh.wp, m.wp);
     }
@@ -1786,7 +1880,8 @@ struct AdjointRun {
         clen = (N + nch0 - 1) / nch0;
         nch = (N + clen - 1) / clen;
         F = (size_t)N * K;
-        const PropShape sh = prop_shape<T>(g, L, RTE_PATH_CACHED, false);  // the forward series'
+        // the forward series'
+        const PropShape sh = prop_shape<T>(g, L, RTE_PATH_CACHED, false, even_medium(grid, m->range, thr));
         if (sh.mfma && (rc = ensure_kexp(m))) return rc;
         HIP_TRY(dW.alloc(F * sizeof(T)));
         HIP_TRY(dWp.alloc(sh.wp * sizeof(T)));
@@ -2397,7 +2492,7 @@ static int propagate_impl(rte_ctx *ctx, rte_medium *m, int L, double prop_thresh
     int rc;
     if ((rc = get_moments(ctx, L, dx, dy, dz, &mom))) return rc;
     if (path == RTE_PATH_CACHED && (rc = ensure_ktab<T>(m, thr))) return rc;
-    const PropShape sh = prop_shape<T>(g, L, path, false);
+    const PropShape sh = prop_shape<T>(g, L, path, false, even_medium(grid, m->range, thr));
     const int nch = sh.nch;
     PropArgs<T> pa;
     std::shared_ptr<DevBuf> zt;
@@ -2811,6 +2906,7 @@ struct ServReq {
     rte_grid grid{};
     std::vector<double> mua, mus, mutd;  // FP64 maps, mu_t = mu_a + mu_s
     std::vector<float> mutf, musf;       // FP32 mu_t, mu_s
+    bool even = false;                   // even_medium
     double g = 0;
     rte_beam beam{};
     int beam_cols = 0;
@@ -2902,7 +2998,7 @@ struct Bucket : BucketBase {
     TA *h_img = nullptr;  // [cap][P]
     std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // by resident count
 
-    Bucket(rte_ctx *c, const rte_grid &gr, const rte_params &pr, int capacity, MomentSet *mom)
+    Bucket(rte_ctx *c, const rte_grid &gr, const rte_params &pr, bool even, int capacity, MomentSet *mom)
         : ctx(c), grid(gr), p(pr)
     {
         cap = capacity;
@@ -2918,7 +3014,7 @@ struct Bucket : BucketBase {
         max_terms = p.max_terms > 0 ? p.max_terms : 1000;
         slot_bytes = rte_solve_footprint(&grid, &p, p.path_mode);
         // the same source chunking as rte_solve_media
-        sh = prop_shape<T>(g, L, p.path_mode, false);
+        sh = prop_shape<T>(g, L, p.path_mode, false, even);
         sc = make_scales(L);
         std::memset(&ca, 0, sizeof ca);
         ca.g = g;
@@ -3210,12 +3306,13 @@ struct rte_server {
     }
 };
 
-static std::string bucket_key(const rte_grid &g, const rte_params &p)
+// (even: of one shape, the solves that the matrix cores take and those that they do not)
+static std::string bucket_key(const rte_grid &g, const rte_params &p, bool even)
 {
     char b[512];
-    snprintf(b, sizeof b, "%d,%d,%d,%.17g,%.17g,%.17g,%.17g,%.17g,%.17g|%d,%d,%d,%.17g,%.17g,%d,%d,%d", g.nx, g.ny, g.nz,
+    snprintf(b, sizeof b, "%d,%d,%d,%.17g,%.17g,%.17g,%.17g,%.17g,%.17g|%d,%d,%d,%.17g,%.17g,%d,%d,%d|%d", g.nx, g.ny, g.nz,
              g.xmin, g.xmax, g.ymin, g.ymax, g.zmin, g.zmax, p.L, p.max_terms, p.stop_rule, p.tol, p.prop_thresh,
-             p.precision, p.exit_quad, p.path_mode);
+             p.precision, p.exit_quad, p.path_mode, even ? 1 : 0);
     return b;
 }
 
@@ -3229,9 +3326,9 @@ static BucketBase *make_bucket(rte_server *S, const ServReq *r, int *rc)
     const int cap = S->opts.max_slots_per_bucket;
     std::unique_ptr<BucketBase> b;
     switch (r->params.precision) {
-    case RTE_PREC_FP64: b.reset(new Bucket<double, double>(S->ctx, gr, r->params, cap, mom)); break;
-    case RTE_PREC_MIXED: b.reset(new Bucket<float, double>(S->ctx, gr, r->params, cap, mom)); break;
-    default: b.reset(new Bucket<float, float>(S->ctx, gr, r->params, cap, mom)); break;
+    case RTE_PREC_FP64: b.reset(new Bucket<double, double>(S->ctx, gr, r->params, r->even, cap, mom)); break;
+    case RTE_PREC_MIXED: b.reset(new Bucket<float, double>(S->ctx, gr, r->params, r->even, cap, mom)); break;
+    default: b.reset(new Bucket<float, float>(S->ctx, gr, r->params, r->even, cap, mom)); break;
     }
     if (b->init_err) {
         *rc = fail(b->init_err, "server: resources for a bucket of %dx%dx%d L=%d", gr.nx, gr.ny, gr.nz,
@@ -3483,7 +3580,10 @@ extern "C" int rte_submit(rte_server *S, const rte_grid *grid, const rte_optics 
     r->g = optics->g;
     r->beam = *beam;
     r->params = *params;
-    r->key = bucket_key(*grid, *params);
+    r->even = params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
+              use_mfma(params->L, make_grid<float>(*grid),
+                       even_medium(*grid, opt_range(optics->mu_a, optics->mu_s, N), params->prop_thresh));
+    r->key = bucket_key(*grid, *params, r->even);
     r->footprint = rte_solve_footprint(grid, params, params->path_mode);
     std::lock_guard<std::mutex> lk(S->mu);
     if (S->failed) return fail(RTE_E_DEVICE, "rte_submit: the server stopped after a device error");

@@ -98,6 +98,7 @@ SIGNATURES = {
     "rte_medium_create": (C.c_int, [_vp, C.POINTER(Grid), C.POINTER(Optics), C.POINTER(_vp)]),
     "rte_medium_destroy": (C.c_int, [_vp]),
     "rte_medium_reset_cache": (C.c_int, [_vp]),
+    "rte_on_matrix_cores": (C.c_int, [_vp, C.POINTER(Params)]),
     "rte_solve_footprint": (C.c_longlong, [C.POINTER(Grid), C.POINTER(Params), C.c_int]),
     "rte_solve": (C.c_int, [_vp, C.POINTER(Grid), C.POINTER(Optics), C.POINTER(Beam),
                             C.POINTER(Params), _dp, C.POINTER(Stats)]),
@@ -233,6 +234,13 @@ class Medium:
 
     def reset_cache(self):
         _check(lib().rte_medium_reset_cache(self.h))
+
+    def on_matrix_cores(self, params):
+        """Whether solves on this medium propagate on the matrix cores (rte_on_matrix_cores)."""
+        rc = lib().rte_on_matrix_cores(self.h, C.byref(params))
+        if rc < 0:
+            _check(rc)
+        return rc == 1
 
     def close(self):
         if self.h:

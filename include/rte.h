@@ -80,6 +80,13 @@ typedef struct {
 #define RTE_PREC_FP64 0  /* everything in FP64 */
 #define RTE_PREC_MIXED 1 /* propagation/scatter FP32; running sums, exitance FP64 */
 #define RTE_PREC_FP32 2  /* everything FP32 */
+/* On large grids at L = 4 and 5 (rte_on_matrix_cores) the cached FP32 propagation of
+ * RTE_PREC_MIXED and RTE_PREC_FP32 multiplies on the FP16 matrix cores: the source's
+ * coefficients, the pair's harmonics and the weighted projections enter as two FP16 pieces
+ * each (22 to 24 bits; 16 neighbouring sources share a power-of-two scale), products are
+ * summed in FP32.  Media where that would keep fewer bits of a voxel's value than FP32 does
+ * (voxels of optical thickness above about 1, couplings cut off within two bricks of 4
+ * voxels, or a cut-off and mu_s over a range of more than 64) stay on FP32 products. */
 
 #define RTE_QUAD_REF 0   /* reference 100-point left Riemann sum (CPU package/src/Dist.c:190-218) */
 #define RTE_QUAD_EXACT 1 /* exact int_0^1 P_l(u) u du */
@@ -154,6 +161,9 @@ int rte_medium_create(rte_ctx *ctx, const rte_grid *grid, const rte_optics *opti
 int rte_medium_destroy(rte_medium *m);
 /* drops the per-medium tables (the next solve rebuilds them) */
 int rte_medium_reset_cache(rte_medium *m);
+/* 1 if solves on this medium propagate on the matrix cores, 0 if not (see RTE_PREC_FP32; it
+ * depends on the medium and params alone, not on what shares a call with the solve), or RTE_E* */
+int rte_on_matrix_cores(const rte_medium *m, const rte_params *params);
 /* bytes of device memory a solve of this shape needs (admission by HBM footprint) */
 long long rte_solve_footprint(const rte_grid *grid, const rte_params *params, int path_mode);
 

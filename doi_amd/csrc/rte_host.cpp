@@ -58,7 +58,7 @@ static int fail(int code, const char *fmt, ...)
 // ---------------------------------------------------------------------------
 // device buffers
 // ---------------------------------------------------------------------------
-static void give_back_tables();  // frees the path tables that contexts keep for reuse
+static void give_back_kept();  // frees the device memory that contexts keep for reuse
 
 struct DevBuf {
     void *p = nullptr;
@@ -81,7 +81,7 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, n);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            give_back_tables();
+            give_back_kept();
             e = hipMalloc(&p, n);
         }
         if (e != hipSuccess) {
@@ -99,26 +99,33 @@ struct DevBuf {
 // A context's path tables (and their exponents) of media that are gone, kept for the next
 // medium of the same size: the driver clears freed memory before it hands it out again, and
 // media made and destroyed with every solve outran it (two tables of 459 MB a 21 ms call:
-// 36 ms).  At most kTablesKeep bytes; given back when an allocation fails and with the
-// context.  A buffer is put here after its context's stream has been synchronized.
+// 36 ms).  At most kTablesKeep bytes, the oldest freed first; given back when an allocation
+// of this library fails, by rte_ctx_trim and with the context.  A buffer is put here after
+// its context's stream has been synchronized.
 constexpr size_t kTablesKeep = size_t(8) << 30;
 struct TablePool {
     std::mutex mu;
-    std::vector<std::pair<void *, size_t>> kept;
+    std::list<std::pair<void *, size_t>> kept;  // oldest first
     size_t bytes = 0;
-    TablePool();
-    ~TablePool();
+    ~TablePool() { give_back(); }
+    void drop_oldest()
+    {
+        (void)hipFree(kept.front().first);
+        bytes -= kept.front().second;
+        kept.pop_front();
+    }
     void put(DevBuf &b)
     {
-        try {
+        if (b.p && b.bytes <= kTablesKeep) {
             std::lock_guard<std::mutex> lk(mu);
-            if (b.p && bytes + b.bytes <= kTablesKeep) {
+            try {
                 kept.emplace_back(b.p, b.bytes);
                 bytes += b.bytes;
                 b.p = nullptr;
                 b.bytes = 0;
+            } catch (const std::bad_alloc &) {  // no room for the list: freed as before
             }
-        } catch (const std::bad_alloc &) {  // no room for the list: freed as before
+            while (bytes > kTablesKeep) drop_oldest();
         }
         b.release();
     }
@@ -128,12 +135,12 @@ struct TablePool {
         b.release();
         {
             std::lock_guard<std::mutex> lk(mu);
-            for (size_t i = 0; i < kept.size(); ++i)
-                if (kept[i].second == n) {
-                    b.p = kept[i].first;
+            for (auto it = kept.begin(); it != kept.end(); ++it)
+                if (it->second == n) {
+                    b.p = it->first;
                     b.bytes = n;
                     bytes -= n;
-                    kept.erase(kept.begin() + i);
+                    kept.erase(it);
                     return hipSuccess;
                 }
         }
@@ -142,31 +149,9 @@ struct TablePool {
     void give_back()
     {
         std::lock_guard<std::mutex> lk(mu);
-        for (auto &k : kept) (void)hipFree(k.first);
-        kept.clear();
-        bytes = 0;
+        while (!kept.empty()) drop_oldest();
     }
 };
-static std::mutex g_pools_mu;
-static std::set<TablePool *> g_pools;
-TablePool::TablePool()
-{
-    std::lock_guard<std::mutex> lk(g_pools_mu);
-    g_pools.insert(this);
-}
-TablePool::~TablePool()
-{
-    {
-        std::lock_guard<std::mutex> lk(g_pools_mu);
-        g_pools.erase(this);
-    }
-    give_back();
-}
-static void give_back_tables()
-{
-    std::lock_guard<std::mutex> lk(g_pools_mu);
-    for (TablePool *p : g_pools) p->give_back();
-}
 
 // Pinned host memory that kernels write their results to (kept, grown as needed): a small
 // copy back costs a launch of the runtime's copy kernel and its staging, ~10 us each; with
@@ -440,7 +425,23 @@ struct rte_ctx {
     DevBuf ws_W, ws_Wp, ws_part, ws_pix, ws_sv, ws_beams;
     std::set<rte_medium *> media;  // live media of this context
     PinBuf pin_red, pin_img;  // sums of a term, images of a batch
+    // frees the path tables of gone media and the Z tables that no call uses
+    void give_back()
+    {
+        tables.give_back();
+        std::lock_guard<std::mutex> lk(ztabs_mu);
+        ztabs.remove_if([](const ZTab &z) { return z.buf.use_count() == 1; });
+    }
 };
+
+// the contexts there are: an allocation that fails, in any thread, takes what all of them keep
+static std::mutex g_ctxs_mu;
+static std::set<rte_ctx *> g_ctxs;
+static void give_back_kept()
+{
+    std::lock_guard<std::mutex> lk(g_ctxs_mu);
+    for (rte_ctx *c : g_ctxs) c->give_back();
+}
 
 // What the choice of the propagation looks at in a medium
 struct OptRange {
@@ -584,6 +585,12 @@ extern "C" int rte_ctx_create(int device, rte_ctx **out)
     HIP_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&ctx->ev0));
     HIP_TRY(hipEventCreate(&ctx->ev1));
+    try {
+        std::lock_guard<std::mutex> lk(g_ctxs_mu);
+        g_ctxs.insert(ctx.get());
+    } catch (const std::bad_alloc &) {
+        return fail(RTE_E_NOMEM, "rte_ctx_create: out of memory");
+    }
     *out = ctx.release();
     return RTE_OK;
 }
@@ -593,6 +600,14 @@ extern "C" int rte_ctx_set_group_size(rte_ctx *ctx, int max_rhs)
     if (!ctx) return fail(RTE_E_ARG, "rte_ctx_set_group_size: NULL");
     if (max_rhs < 1 || max_rhs > kMaxNR) return fail(RTE_E_ARG, "group size %d outside 1..%d", max_rhs, kMaxNR);
     ctx->max_rhs = max_rhs;
+    return RTE_OK;
+}
+
+extern "C" int rte_ctx_trim(rte_ctx *ctx)
+{
+    if (!ctx) return fail(RTE_E_ARG, "rte_ctx_trim: NULL");
+    (void)hipSetDevice(ctx->device);
+    ctx->give_back();
     return RTE_OK;
 }
 
@@ -631,6 +646,10 @@ extern "C" int rte_ctx_destroy(rte_ctx *ctx)
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    {
+        std::lock_guard<std::mutex> lk(g_ctxs_mu);
+        g_ctxs.erase(ctx);
+    }
     delete ctx;
     return RTE_OK;
 }
@@ -805,6 +824,7 @@ static int ensure_ktab(rte_medium *m, double thr, hipStream_t on = nullptr)
     if (tab.p && tthr == thr) return RTE_OK;
     const GridDev<T> g = make_grid<T>(m->grid);
     if (sizeof(T) == 4) m->kexp_ok = false;
+    tthr = NAN;  // nothing is in the table until its launch has been made
     HIP_TRY(m->ctx->tables.get(tab, (size_t)g.N * g.npad * sizeof(T)));
     const T *mut = sizeof(T) == 4 ? (const T *)m->mut_f.p : (const T *)m->mut_d.p;
     const T thr2 = thr > 0 ? T(thr * thr) : T(sizeof(T) == 4 ? 1e30 : 1e300);
@@ -923,17 +943,26 @@ static int get_ztab(rte_ctx *ctx, int L, const GridDev<float> &g, double dx, dou
                     std::shared_ptr<DevBuf> *out)
 {
     const auto key = std::make_tuple(L, g.bx, g.by, g.nz, dx, dy, dz);
-    std::lock_guard<std::mutex> lk(ctx->ztabs_mu);
-    for (auto it = ctx->ztabs.begin(); it != ctx->ztabs.end(); ++it)
-        if (it->key == key) {
-            ctx->ztabs.splice(ctx->ztabs.begin(), ctx->ztabs, it);
-            *out = it->buf;
-            return RTE_OK;
-        }
+    auto find = [&] {
+        for (auto it = ctx->ztabs.begin(); it != ctx->ztabs.end(); ++it)
+            if (it->key == key) {
+                ctx->ztabs.splice(ctx->ztabs.begin(), ctx->ztabs, it);
+                *out = it->buf;
+                return true;
+            }
+        return false;
+    };
+    {
+        std::lock_guard<std::mutex> lk(ctx->ztabs_mu);
+        if (find()) return RTE_OK;
+    }
+    // made outside the lock, which an allocation that fails takes to give back the others
     auto buf = std::make_shared<DevBuf>();
     HIP_TRY(buf->alloc(mfma_ztab_bytes(L, g)));
     HIP_TRY(launch_ztab(L, g, dx, dy, dz, buf->as<unsigned char>(), st));
     HIP_TRY(hipStreamSynchronize(st));  // other streams may use it next
+    std::lock_guard<std::mutex> lk(ctx->ztabs_mu);
+    if (find()) return RTE_OK;
     ctx->ztabs.push_front(ZTab{key, buf});
     size_t kept = 0;
     for (auto it = ctx->ztabs.begin(); it != ctx->ztabs.end();) {
@@ -3514,7 +3543,7 @@ extern "C" int rte_server_create(rte_ctx *ctx, const rte_server_opts *opts, rte_
     if (S->opts.hbm_budget <= 0) {
         size_t fr = 0, tot = 0;
         HIP_TRY(hipSetDevice(ctx->device));
-        give_back_tables();  // kept memory counts as free
+        give_back_kept();  // kept memory counts as free
         HIP_TRY(hipMemGetInfo(&fr, &tot));
         S->opts.hbm_budget = (long long)(0.8 * (double)fr);
     }

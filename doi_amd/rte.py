@@ -92,6 +92,7 @@ SIGNATURES = {
     "rte_last_error": (C.c_char_p, []),
     "rte_ctx_create": (C.c_int, [C.c_int, C.POINTER(_vp)]),
     "rte_ctx_destroy": (C.c_int, [_vp]),
+    "rte_ctx_trim": (C.c_int, [_vp]),
     "rte_ctx_profile": (C.c_int, [_vp, C.c_int]),
     "rte_ctx_set_group_size": (C.c_int, [_vp, C.c_int]),
     "rte_ctx_get_profile": (C.c_int, [_vp, C.POINTER(Prof)]),
@@ -280,6 +281,10 @@ class Context:
 
     def set_group_size(self, max_rhs):
         _check(lib().rte_ctx_set_group_size(self.h, max_rhs))
+
+    def trim(self):
+        """Gives back the device memory that the context keeps for later calls (rte_ctx_trim)."""
+        _check(lib().rte_ctx_trim(self.h))
 
     def profile(self, on=True):
         _check(lib().rte_ctx_profile(self.h, 1 if on else 0))

@@ -147,6 +147,12 @@ int rte_ctx_destroy(rte_ctx *ctx);
  * medium share a propagation launch on the mixed-precision cached path (by default 16
  * solves where it runs on the matrix cores); the result bits do not depend on it */
 int rte_ctx_set_group_size(rte_ctx *ctx, int max_rhs);
+/* gives the device back what the context keeps for later calls: the path tables of gone
+ * and reset media (at most 8 GiB, for media of the same size) and the displacement tables
+ * of grids that ran on the matrix cores (at most 1 GiB).  This library's own allocations
+ * take them when they fail, and rte_server_create when it sizes itself by the free memory;
+ * for other users of the device's memory, call this. */
+int rte_ctx_trim(rte_ctx *ctx);
 /* on != 0: time every launch from now on (resets the counters); 0: stop */
 int rte_ctx_profile(rte_ctx *ctx, int on);
 int rte_ctx_get_profile(rte_ctx *ctx, rte_prof *out);
@@ -158,8 +164,10 @@ int rte_version(void);
  * its per-medium tables (path integrals, self blocks) across calls. */
 int rte_medium_create(rte_ctx *ctx, const rte_grid *grid, const rte_optics *optics,
                       rte_medium **out);
+/* (the context keeps the memory of its path tables: rte_ctx_trim) */
 int rte_medium_destroy(rte_medium *m);
-/* drops the per-medium tables (the next solve rebuilds them) */
+/* drops the per-medium tables (the next solve rebuilds them; their memory as with
+ * rte_medium_destroy) */
 int rte_medium_reset_cache(rte_medium *m);
 /* 1 if solves on this medium propagate on the matrix cores, 0 if not (see RTE_PREC_FP32; it
  * depends on the medium and params alone, not on what shares a call with the solve), or RTE_E* */

@@ -780,15 +780,10 @@ static hipError_t launch_bp_as(const GridDev<T> &g, BpPlan p, size_t lds, int cu
 template <typename T, typename TA>
 hipError_t launch_backproject(const GridDev<T> &g, T thr2, const T *pairbuf, TA scale, TA *gt, hipStream_t st)
 {
-    static int lds_max = -1, cus = 0;
-    if (lds_max < 0) {
-        int dev = 0, v = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-        if (e != hipSuccess) return e;
-        lds_max = v;
-    }
+    DevLimits lim;
+    const hipError_t le = device_limits(&lim);
+    if (le != hipSuccess) return le;
+    const int lds_max = lim.lds_max, cus = lim.cus;
     // odd pitches (the translations' voxels in different banks) where that fits
     BpPlan p{};
     size_t lds = 0;
@@ -821,14 +816,10 @@ hipError_t launch_backproject(const GridDev<T> &g, T thr2, const T *pairbuf, TA 
 template <typename T, typename TA>
 hipError_t launch_backproject_blocks(const GridDev<T> &g, T thr2, const BlockBp<T, TA> &B, int nc, hipStream_t st)
 {
-    static int lds_max = -1;
-    if (lds_max < 0) {
-        int dev = 0, v = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-        if (e != hipSuccess) return e;
-        lds_max = v;
-    }
+    DevLimits lim;
+    const hipError_t le = device_limits(&lim);
+    if (le != hipSuccess) return le;
+    const int lds_max = lim.lds_max;
     if (nc < 1 || nc > kMaxNC || B.nparam < 1) return hipErrorInvalidValue;
     const size_t lds = (((size_t)g.N * sizeof(int) + 15) & ~size_t(15)) + (size_t)nc * B.nparam * sizeof(TA);
     if (lds > (size_t)lds_max) return hipErrorInvalidValue;  // the caller back-projects per voxel

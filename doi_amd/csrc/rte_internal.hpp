@@ -145,6 +145,11 @@ hipError_t launch_prop_sep(int L, int nr, const PropArgs<T> &A, const SolveDev<T
 template <typename T, typename TA>
 hipError_t launch_prop_c(int L, int path, const PropArgs<T> &A, const SolveDev<T, TA> *sv, int ncomplex,
                          hipStream_t st);
+// of the current device, asked for once a device, from any thread: LDS bytes a block can have, CUs
+struct DevLimits {
+    int lds_max = 0, cus = 0;
+};
+hipError_t device_limits(DevLimits *out);
 // matrix-core propagation (rte_mfma.hip), A.zt set: ngroups * nr solves on any media of one
 // grid, their W first brought into pieces; each solve's Wp holds mfma_wp_bytes
 size_t mfma_wp_bytes(int L, const GridDev<float> &g);

@@ -22,6 +22,8 @@
 // on how many solves share a launch.
 #include "rte_device.hpp"
 
+#include <mutex>
+
 namespace rte {
 
 template <typename T>
@@ -1313,6 +1315,28 @@ hipError_t launch_prop_c(int L, int path, const PropArgs<T> &A, const SolveDev<T
     return hipGetLastError();
 }
 
+hipError_t device_limits(DevLimits *out)
+{
+    constexpr int most = 64;
+    static std::mutex mu;
+    static DevLimits known[most];
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= most) return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> lk(mu);
+    DevLimits &d = known[dev];
+    if (!d.cus) {
+        DevLimits v;
+        e = hipDeviceGetAttribute(&v.cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&v.lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+        if (e != hipSuccess) return e;
+        d = v;
+    }
+    *out = d;
+    return hipSuccess;
+}
+
 template <typename T, int MEM, int M, int SG, int THREADS>
 static hipError_t launch_ktab_as(const GridDev<T> &g, KtabPlan p, size_t lds, int cus, T thr2, const T *mut, T *ktab,
                                  hipStream_t st)
@@ -1332,15 +1356,10 @@ static hipError_t launch_ktab_as(const GridDev<T> &g, KtabPlan p, size_t lds, in
 template <typename T>
 hipError_t launch_ktab(const GridDev<T> &g, T thr2, const T *mut, T *ktab, hipStream_t st)
 {
-    static int lds_max = -1, cus = 0;
-    if (lds_max < 0) {
-        int dev = 0, v = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-        if (e != hipSuccess) return e;
-        lds_max = v;
-    }
+    DevLimits lim;
+    const hipError_t e = device_limits(&lim);
+    if (e != hipSuccess) return e;
+    const int lds_max = lim.lds_max, cus = lim.cus;
     // LDS pitches: y = 4 (mod 8), z = 16 (mod 32) put the 64 voxels of a brick in
     // different banks (5 % at 24^3 and 32^3); the plain map where that does not fit
     KtabPlan p{};

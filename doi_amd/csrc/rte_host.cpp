@@ -1516,6 +1516,12 @@ static int check_params(const rte_params *p)
     return RTE_OK;
 }
 
+static bool on_matrix_cores(const rte_grid &grid, const rte_params &p, const OptRange &r)
+{
+    return p.precision != RTE_PREC_FP64 && p.path_mode == RTE_PATH_CACHED &&
+           use_mfma(p.L, make_grid<float>(grid), even_medium(grid, r, p.prop_thresh));
+}
+
 static int solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
                         const rte_params *params, double *exitance, double *reflectance, rte_stats *stats)
 {
@@ -1548,11 +1554,8 @@ extern "C" int rte_solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, 
     }
     if ((rc = set_device(ctx))) return rc;
     // solves that the matrix cores take and solves that they do not are batches of their own
-    const GridDev<float> g = make_grid<float>(media[0]->grid);
     std::vector<int> on, off;
-    if (params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED && use_mfma(params->L, g, true))
-        for (int i = 0; i < nb; ++i)
-            (even_medium(media[i]->grid, media[i]->range, params->prop_thresh) ? on : off).push_back(i);
+    for (int i = 0; i < nb; ++i) (on_matrix_cores(media[i]->grid, *params, media[i]->range) ? on : off).push_back(i);
     if (on.empty() || off.empty()) return solve_images(ctx, nb, media, beams, params, exitance, reflectance, stats);
     const size_t P = (size_t)media[0]->grid.nx * media[0]->grid.ny;
     double gpu_ms = 0.0;
@@ -1823,30 +1826,28 @@ extern "C" int rte_on_matrix_cores(const rte_medium *m, const rte_params *params
     if (!m) return fail(RTE_E_ARG, "rte_on_matrix_cores: NULL medium");
     int rc;
     if ((rc = check_params(params))) return rc;
-    return params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
-           use_mfma(params->L, make_grid<float>(m->grid), even_medium(m->grid, m->range, params->prop_thresh));
+    return on_matrix_cores(m->grid, *params, m->range);
+}
+
+// device memory of one solve of a shape; on: it propagates on the matrix cores
+static long long solve_bytes(const rte_grid &grid, const rte_params &p, int path_mode, bool on)
+{
+    const GridDev<float> g = make_grid<float>(grid);
+    const long long K = (p.L + 1) * (p.L + 1), N = g.N;
+    const long long es = p.precision == RTE_PREC_FP64 ? 8 : 4;
+    const PropShape sh = prop_shape<float>(g, p.L, on ? RTE_PATH_CACHED : RTE_PATH_MARCH, false, true);
+    long long bytes = N * 8 * 3 + N * 4 * 2;                    // maps
+    bytes += N * K * es * (1 + sh.nch) + (long long)sh.wp * es;  // W, partials, the propagation's copy of W
+    bytes += (long long)grid.nx * grid.ny * kPixBufs * 8 + 64;   // pixel buffers
+    if (path_mode == RTE_PATH_CACHED) bytes += N * (long long)g.npad * es;
+    if (sh.mfma) bytes += (long long)kexp_bytes(g);
+    return bytes;
 }
 
 extern "C" long long rte_solve_footprint(const rte_grid *grid, const rte_params *params, int path_mode)
 {
     if (!grid || !params || params->L < 0 || params->L > RTE_MAX_L) return -1;
-    const GridDev<float> g = make_grid<float>(*grid);
-    const long long K = (params->L + 1) * (params->L + 1);
-    const long long es = params->precision == RTE_PREC_FP64 ? 8 : 4;
-    const long long N = g.N;
-    // the larger of the shapes that solves of this grid and order take; the 1/64 of a path table
-    // that the matrix cores' exponents take, and the Z table that a grid's solves share, not counted
-    PropShape sh = prop_shape<float>(g, params->L, RTE_PATH_MARCH, false, true);
-    if (params->precision != RTE_PREC_FP64) {
-        const PropShape m = prop_shape<float>(g, params->L, RTE_PATH_CACHED, false, true);
-        sh.nch = std::max(sh.nch, m.nch);
-        sh.wp = std::max(sh.wp, m.wp);
-    }
-    long long bytes = N * 8 * 3 + N * 4 * 2;             // maps
-    bytes += N * K * es * (1 + sh.nch) + (long long)sh.wp * es;  // W, partials, the propagation's copy of W
-    bytes += (long long)grid->nx * grid->ny * kPixBufs * 8 + 64; // pixel buffers
-    if (path_mode == RTE_PATH_CACHED) bytes += N * (long long)g.npad * es;
-    return bytes;
+    return solve_bytes(*grid, *params, path_mode, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -2935,7 +2936,7 @@ struct ServReq {
     rte_grid grid{};
     std::vector<double> mua, mus, mutd;  // FP64 maps, mu_t = mu_a + mu_s
     std::vector<float> mutf, musf;       // FP32 mu_t, mu_s
-    bool even = false;                   // even_medium
+    bool on = false;                     // the matrix cores propagate
     double g = 0;
     rte_beam beam{};
     int beam_cols = 0;
@@ -3027,7 +3028,7 @@ struct Bucket : BucketBase {
     TA *h_img = nullptr;  // [cap][P]
     std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // by resident count
 
-    Bucket(rte_ctx *c, const rte_grid &gr, const rte_params &pr, bool even, int capacity, MomentSet *mom)
+    Bucket(rte_ctx *c, const rte_grid &gr, const rte_params &pr, bool on, int capacity, MomentSet *mom)
         : ctx(c), grid(gr), p(pr)
     {
         cap = capacity;
@@ -3041,9 +3042,9 @@ struct Bucket : BucketBase {
         dz = (grid.zmax - grid.zmin) / grid.nz;
         thr = p.prop_thresh > 0 ? p.prop_thresh : -1.0;
         max_terms = p.max_terms > 0 ? p.max_terms : 1000;
-        slot_bytes = rte_solve_footprint(&grid, &p, p.path_mode);
+        slot_bytes = solve_bytes(grid, p, p.path_mode, on);
         // the same source chunking as rte_solve_media
-        sh = prop_shape<T>(g, L, p.path_mode, false, even);
+        sh = prop_shape<T>(g, L, p.path_mode, false, on);
         sc = make_scales(L);
         std::memset(&ca, 0, sizeof ca);
         ca.g = g;
@@ -3335,13 +3336,13 @@ struct rte_server {
     }
 };
 
-// (even: of one shape, the solves that the matrix cores take and those that they do not)
-static std::string bucket_key(const rte_grid &g, const rte_params &p, bool even)
+// (on: of one shape, the solves that the matrix cores take and those that they do not)
+static std::string bucket_key(const rte_grid &g, const rte_params &p, bool on)
 {
     char b[512];
     snprintf(b, sizeof b, "%d,%d,%d,%.17g,%.17g,%.17g,%.17g,%.17g,%.17g|%d,%d,%d,%.17g,%.17g,%d,%d,%d|%d", g.nx, g.ny, g.nz,
              g.xmin, g.xmax, g.ymin, g.ymax, g.zmin, g.zmax, p.L, p.max_terms, p.stop_rule, p.tol, p.prop_thresh,
-             p.precision, p.exit_quad, p.path_mode, even ? 1 : 0);
+             p.precision, p.exit_quad, p.path_mode, on ? 1 : 0);
     return b;
 }
 
@@ -3355,9 +3356,9 @@ static BucketBase *make_bucket(rte_server *S, const ServReq *r, int *rc)
     const int cap = S->opts.max_slots_per_bucket;
     std::unique_ptr<BucketBase> b;
     switch (r->params.precision) {
-    case RTE_PREC_FP64: b.reset(new Bucket<double, double>(S->ctx, gr, r->params, r->even, cap, mom)); break;
-    case RTE_PREC_MIXED: b.reset(new Bucket<float, double>(S->ctx, gr, r->params, r->even, cap, mom)); break;
-    default: b.reset(new Bucket<float, float>(S->ctx, gr, r->params, r->even, cap, mom)); break;
+    case RTE_PREC_FP64: b.reset(new Bucket<double, double>(S->ctx, gr, r->params, r->on, cap, mom)); break;
+    case RTE_PREC_MIXED: b.reset(new Bucket<float, double>(S->ctx, gr, r->params, r->on, cap, mom)); break;
+    default: b.reset(new Bucket<float, float>(S->ctx, gr, r->params, r->on, cap, mom)); break;
     }
     if (b->init_err) {
         *rc = fail(b->init_err, "server: resources for a bucket of %dx%dx%d L=%d", gr.nx, gr.ny, gr.nz,
@@ -3609,11 +3610,9 @@ extern "C" int rte_submit(rte_server *S, const rte_grid *grid, const rte_optics 
     r->g = optics->g;
     r->beam = *beam;
     r->params = *params;
-    r->even = params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
-              use_mfma(params->L, make_grid<float>(*grid),
-                       even_medium(*grid, opt_range(optics->mu_a, optics->mu_s, N), params->prop_thresh));
-    r->key = bucket_key(*grid, *params, r->even);
-    r->footprint = rte_solve_footprint(grid, params, params->path_mode);
+    r->on = on_matrix_cores(*grid, *params, opt_range(optics->mu_a, optics->mu_s, N));
+    r->key = bucket_key(*grid, *params, r->on);
+    r->footprint = solve_bytes(*grid, *params, params->path_mode, r->on);
     std::lock_guard<std::mutex> lk(S->mu);
     if (S->failed) return fail(RTE_E_DEVICE, "rte_submit: the server stopped after a device error");
     if (r->footprint > S->opts.hbm_budget)

@@ -597,26 +597,32 @@ def main():
     value = nsolve / (ms_per_step / 1000.0)
     terms_mean = float(np.mean([s["terms"] for s in stats]))
 
-    # roofline of the dominant kernel: k_prop_mfma on the grids and orders that the library
-    # runs on the matrix cores (groups of five and more beams counted under 5), else the
-    # propagation group of the default size (k_prop<float, double, L, 0, 5>; the library
-    # allows at most 3 at L = 6 and 2 from L = 7): its algorithmic flops / its launch time
-    on_mfma = L in (4, 5) and n >= 32
+    # roofline of the dominant kernel: where the library propagates on the matrix cores
+    # k_prop_mfma, all of its launches (groups of up to 16 solves); else the propagation group of
+    # the default size (k_prop<float, double, L, 0, 5>; the library allows at most 3 at L = 6 and
+    # 2 from L = 7): its algorithmic flops / its launch time
+    on_mfma = all(m.on_matrix_cores(prm) for m in mm)
+    K = (L + 1) ** 2
+    npairs = float(n ** 3) * (n ** 3 - 1)
     gsz = min(args.group or DEFAULT_GROUP, args.beams, 5 if L <= 5 else (3 if L == 6 else 2))
-    launches = max(prof["group_launches"][gsz], 1)
-    avg_ms = prof["group_ms"][gsz] / launches
-    flops_per_launch = prof["group_flops"][gsz] / launches
-    achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
     pairs_per_s = prof["prop_pairs"] / (prof["prop_ms"] * 1e-3) if prof["prop_ms"] > 0 else 0.0
     all_launches = max(prof["prop_launches"], 1)
     achieved_all = prof["prop_flops"] / (prof["prop_ms"] * 1e-3) / 1e12 if prof["prop_ms"] > 0 else 0.0
-    K = (L + 1) ** 2
-    npairs = float(n ** 3) * (n ** 3 - 1)
-    # beam-terms a launch processes: the library counts (16 + k 4K) flops per pair of a group of k
-    beam_terms = flops_per_launch / ((16 + gsz * 4 * K) * npairs) * gsz
-    # the matrix flops that k_prop_mfma executes: FP16 products of two pieces each, 10 (L = 4: 7)
-    # of 16 x 16 x 32 per 16 sources x 16 destinations x 16 columns and source (or destination)
-    executed = achieved * (10 if L == 5 else 7) * 64.0 / (4 * K)
+    if on_mfma:
+        launches, avg_ms = all_launches, prof["prop_ms"] / all_launches
+        flops_per_launch, achieved = prof["prop_flops"] / all_launches, achieved_all
+        beam_terms = prof["prop_pairs"] / all_launches / npairs
+        # FP16 products of two pieces, 64 flops per pair and solve each: 3 of the projection's 32
+        # coefficients and 4 of the sums' (L = 4: 25 of 32 used), at L = 5 the last 4 coefficients'
+        # in half of one and a quarter of two more (the padding of either is not counted)
+        executed = pairs_per_s * 64.0 * (8.0 if L == 5 else 7.0 * 25 / 32) / 1e12
+    else:
+        launches = max(prof["group_launches"][gsz], 1)
+        avg_ms = prof["group_ms"][gsz] / launches
+        flops_per_launch = prof["group_flops"][gsz] / launches
+        executed = achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
+        # beam-terms a launch processes: the library counts (16 + k 4K) flops per pair of a group of k
+        beam_terms = flops_per_launch / ((16 + gsz * 4 * K) * npairs) * gsz
     peak = PEAK_F16_MFMA_TFLOPS if on_mfma else PEAK_FP32_TFLOPS
     traffic = None
     if n == 32 and L == 5 and gsz in TRAFFIC_PER_SOLVE_TERM and not on_mfma:
@@ -665,7 +671,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "fp32 (fp64 running sums)",
+        "dtype": "fp32 (fp64 running sums%s)" % ("; propagation factors as two fp16 pieces each" if on_mfma else ""),
         "data": "synthetic (seeded lognormal media with inclusions)",
         "config": {"workload": "%d lognormal media with inclusions x %d beams, %d^3 voxels 0.1 cm, L=%d, g=0.9, tol 1e-6 cap 30"
                                % (args.media, args.beams, n, L),
@@ -678,17 +684,17 @@ def main():
         "terms_mean": terms_mean,
         "voxel_pair_propagations_per_s": pairs_per_s,
         "roofline": {"bound": "mfma" if on_mfma else "valu", "pipe": "mfma-f16" if on_mfma else "valu-fp32",
-                     "achieved": executed if on_mfma else achieved, "peak": peak,
-                     "unit": "TFLOP/s", "frac": (executed if on_mfma else achieved) / peak, "traffic": traffic,
+                     "achieved": executed, "peak": peak,
+                     "unit": "TFLOP/s", "frac": executed / peak, "traffic": traffic,
                      "algorithmic_tflops": achieved,
-                     "kernel": "k_prop_mfma<double, %d> (groups of five and more solves, cached path)" % L if on_mfma else
+                     "kernel": "k_prop_mfma<double, %d> (groups of up to 16 solves, cached path)" % L if on_mfma else
                                "k_prop<float, double, %d, 0, %d> (groups of %d beams, cached path)" % (L, gsz, gsz),
                      "launches": launches, "avg_launch_ms": avg_ms, "flops_per_launch": flops_per_launch,
                      "beam_terms_per_launch": beam_terms,
                      "all_propagation_launches": {"launches": all_launches,
                                                   "avg_launch_ms": prof["prop_ms"] / all_launches,
                                                   "achieved": achieved_all,
-                                                  "frac": achieved_all / PEAK_FP32_TFLOPS}},
+                                                  "frac": None if on_mfma else achieved_all / PEAK_FP32_TFLOPS}},
     }
     res.update(out)
     res["ktab_ms_total"] = prof["ktab_ms"]

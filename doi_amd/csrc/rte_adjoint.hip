@@ -389,24 +389,28 @@ __global__ void k_make_wq(GridDev<T> g, Scales sc, TA gan, const T *mus, const T
 // only the pairs with slot(s) < slot(d).
 // A wave takes M translations of a brick pair, lane = (translation, 64 / M of the
 // destinations), and walks 16 sources of the brick with M steps over its
-// destinations.  With the 64 destinations of one source in a wave (the layout before
-// this) the rays leave the source through the same few voxels, and the atomics on
+// destinations; what lies beyond the grid for all its translations is left out.  With
+// M = 1 its rays leave the source through the same few voxels, and the atomics on
 // one address are served one after the other, ~110 clocks of the LDS per crossing;
-// translated rays are in different voxels throughout.  24^3 (FP64 sums) before 9.0,
-// now 3.7 ms.
+// translated rays are in different voxels throughout, but a small grid has few
+// translations, and a ragged one leaves lanes without a voxel: see launch_backproject.
 // A grid whose sums do not fit the LDS goes in slabs of z planes, a y-row of blocks each:
 // a slab's rays (those that reach it) are walked whole and their voxels outside it left
 // out.  (With atomics in memory a gradient at
 // 28^3, L = 5, 8 terms took 506 ms, 32^3 1302, 40^3, L = 3, 5139; in slabs 55, 92 and 310.)  Only where that takes
 // more than kBpSlabs slabs do the atomics go to memory.
-// grid = (at most the resident blocks, slabs); unit u (translation group, D, 16 of the
-// source brick's 64 voxels) belongs to block u mod grid, whose waves share its units.
+// grid = (at most the resident blocks, slabs); of the units (translation group, D, 16 of
+// the source brick's 64 voxels) a block takes one of each run of gridDim.x, its waves
+// share them.  Which one moves on by rot from run to run where the z planes of a brick
+// are not all in the grid: with the same one, 3 of 4 blocks of a grid of one plane had
+// nothing to do (100x100x1: 18.6 -> 4.5 ms).
 // ---------------------------------------------------------------------------
 constexpr int kBpSlabs = 16;
 struct BpPlan {
     int py, pz;      // pitches of y and z in the accumulator (elements)
     int zs;          // z planes of a slab
     int nD, nunits;
+    int rot;
     int next;        // where in LDS the block's unit counter lies (bytes), -1: no room
 };
 
@@ -432,8 +436,10 @@ __global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, BpPlan p
     for (int own = tid / kWave;; own += blockDim.x / kWave) {
         // the block's next unit (in a fixed order where the accumulator leaves no room for a counter)
         if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
-        const int u = blockIdx.x + gridDim.x * __builtin_amdgcn_readfirstlane(own);
-        if (u >= p.nunits) break;
+        const unsigned run = __builtin_amdgcn_readfirstlane(own);
+        const int u = (int)((blockIdx.x + run * (unsigned)p.rot) % gridDim.x + gridDim.x * run);
+        if (gridDim.x * run >= (unsigned)p.nunits) break;
+        if (u >= p.nunits) continue;
         const int slab = u & 3, f = (u >> 2) % p.nD + p.nD - 1, first = (u >> 2) / p.nD * M;
         const int Dx = f % ex - (g.bx - 1), Dy = (f / ex) % ey - (g.by - 1), Dz = f / (ex * ey) - (g.bz - 1);
         const int cx = g.bx - abs(Dx), cy = g.by - abs(Dy), cnt = cx * cy * (g.bz - abs(Dz));
@@ -443,6 +449,34 @@ __global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, BpPlan p
         const int t = min(first + m, cnt - 1);
         const int bx0 = t % cx + max(0, -Dx), by0 = (t / cx) % cy + max(0, -Dy), bz0 = t / (cx * cy) + max(0, -Dz);
         const int bs = bx0 + g.bx * (by0 + g.by * bz0), bd = bs + Dx + g.bx * (Dy + g.by * Dz);
+        // the nearest pair of the bricks is not coupled (thr2 is rounded, and r^2 below)
+        const T nearx = T(max(0, kBrick * abs(Dx) - 3)) * g.dx, neary = T(max(0, kBrick * abs(Dy) - 3)) * g.dy,
+                nearz = T(max(0, kBrick * abs(Dz) - 3)) * g.dz;
+        if (sum_squares(nearx, neary, nearz) > thr2 * T(1.0001)) continue;
+        // the lowest voxels of the wave's source bricks: a source (or the part of the destinations
+        // that the step alone decides) that is beyond the grid there is so for all of them
+        int lx = bx0, ly = by0, lz = bz0;
+        if constexpr (M > 1) {
+#pragma unroll
+            for (int o = kWave / 2; o >= ND; o >>= 1) {
+                lx = min(lx, __shfl_xor(lx, o));
+                ly = min(ly, __shfl_xor(ly, o));
+                lz = min(lz, __shfl_xor(lz, o));
+            }
+        }
+        lx = __builtin_amdgcn_readfirstlane(lx) * kBrick;
+        ly = __builtin_amdgcn_readfirstlane(ly) * kBrick;
+        lz = __builtin_amdgcn_readfirstlane(lz) * kBrick;
+        auto from = [&](int it) {  // the first step from it on with a pair in the grid
+            for (; it < 16 * M; ++it) {
+                const int q = slab * 16 + it / M, j = it % M * ND;
+                if (lx + (q & 3) < g.nx && ly + ((q >> 2) & 3) < g.ny && lz + (q >> 4) < g.nz &&
+                    (ND >= 16 || ly + Dy * kBrick + ((j >> 2) & 3) < g.ny) &&
+                    (ND >= 64 || lz + Dz * kBrick + (j >> 4) < g.nz))
+                    break;
+            }
+            return it;
+        };
         // pair it = source 16 slab + it / M of the brick, destination slot (it % M) ND + sub
         struct Pair { int ix, iy, iz, v; T r2, w0, w1; };
         auto load = [&](int it) {
@@ -466,10 +500,13 @@ __global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, BpPlan p
             }
             return P;
         };
-        Pair nx = load(0);
-        for (int it = 0; it < 16 * M; ++it) {
+        int it = from(0);
+        if (it == 16 * M) continue;
+        Pair nx = load(it);
+        while (it < 16 * M) {
             const Pair P = nx;
-            if (it + 1 < 16 * M) nx = load(it + 1);  // the next pair's weights under this one's march
+            it = from(it + 1);
+            if (it < 16 * M) nx = load(it);  // the next pair's weights under this one's march
             const TA w = TA(P.w0) + TA(P.w1);
             if (w == TA(0)) continue;
             const TA sw = scale * w;
@@ -767,10 +804,13 @@ static hipError_t launch_bp_as(const GridDev<T> &g, BpPlan p, size_t lds, int cu
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    // a large accumulator leaves room for one block per CU: make it 16 waves
-    const int threads = lds > 64 * 1024 ? 1024 : 256, waves = threads / kWave;
+    // a large accumulator leaves room for one block per CU: make it 16 waves.  M = 1 takes as
+    // many as fit (18^3, 47 KB: 24 waves a CU 1.10 ms, 12 1.36)
+    const int threads = lds > 64 * 1024 ? 1024 : M == 1 ? 512 : 256, waves = threads / kWave;
+    const int percu = M == 1 && threads == 512 ? min(4, (int)(160 * 1024 / lds)) : 1024 / threads;
     p.nunits = p.nD * ((g.nblk + M - 1) / M) * 4;
-    const int blocks = min((p.nunits + waves - 1) / waves, cus * (1024 / threads));
+    const int blocks = min((p.nunits + waves - 1) / waves, cus * percu);
+    p.rot = g.nz % kBrick ? (int)(0.618 * blocks) | 1 : 0;
     const int slabs = MEM == 2 ? (g.nz + p.zs - 1) / p.zs : 1;
     hipLaunchKernelGGL((k_backproject_sym<T, TA, MEM, M>), dim3(blocks, slabs), dim3(threads), lds, st, g, p, thr2, pairbuf,
                        scale, gt);
@@ -804,11 +844,31 @@ hipError_t launch_backproject(const GridDev<T> &g, T thr2, const T *pairbuf, TA 
         lds = 16;
     }
     p.nD = ((2 * g.bx - 1) * (2 * g.by - 1) * (2 * g.bz - 1) + 1) / 2;
-    // 16 translations where most brick displacements have that many, else 4
-    const bool many = g.nblk >= 64;
-#define RTE_BP(MEM)                                                                              \
-    (many ? launch_bp_as<T, TA, MEM, 16>(g, p, lds, cus, thr2, pairbuf, scale, gt, st)           \
-          : launch_bp_as<T, TA, MEM, 4>(g, p, lds, cus, thr2, pairbuf, scale, gt, st))
+    // 16 translations where the crossings are many enough for their units to fill the chip;
+    // 1 on smaller grids, and on thin ones, whose translations meet in the same columns; 4 where a
+    // coupling threshold leaves little of a large grid.  us with 1 / 4 / 16, FP32 table: 8^3 29 /
+    // 127 / 567, 16^3 603 / 710 / 1043, 20^3 2300 / 2580 / 1640, 24^3 7430 / 7680 / 3760 (threshold
+    // of 4.7 voxels 161 / 126 / 296, 10.3 806 / 815 / 667), 100x100x1 11900 / 11100 / 4500, 5x5x200
+    // 2480 / 2740 / 4280; a wave per brick pair and source, as before the translations: 8^3 152,
+    // 16^3 760, 20^3 2290, 24^3 8210, 100x100x1 12300, 5x5x200 3620
+    double cross = 0.0;  // voxels crossed by the coupled pairs' rays
+    const double fill = (double)g.N / g.npad;
+    for (int Dz = 0; Dz < g.bz; ++Dz)
+        for (int Dy = 0; Dy < g.by; ++Dy)
+            for (int Dx = 0; Dx < g.bx; ++Dx) {
+                const double x = (double)kBrick * Dx * g.dx, y = (double)kBrick * Dy * g.dy, z = (double)kBrick * Dz * g.dz;
+                if (x * x + y * y + z * z >= (double)thr2) continue;
+                const double signs = (Dx ? 2.0 : 1.0) * (Dy ? 2.0 : 1.0) * (Dz ? 2.0 : 1.0);
+                cross += 0.5 * signs * (g.bx - Dx) * (g.by - Dy) * (g.bz - Dz) * kBrick * max(1, Dx + Dy + Dz);
+            }
+    cross *= fill * fill * kWave * kWave;
+    const int top = max(g.bx, max(g.by, g.bz));
+    const bool thin = g.nblk < 10 * top, big = g.nblk >= 200;  // 10 bricks a layer across the longest axis
+    const int most = thin ? 1 : cross >= (big ? 1.8e8 : 6e8) ? 16 : big ? 4 : 1;
+#define RTE_BP(MEM)                                                                                   \
+    (most == 16  ? launch_bp_as<T, TA, MEM, 16>(g, p, lds, cus, thr2, pairbuf, scale, gt, st)         \
+     : most == 4 ? launch_bp_as<T, TA, MEM, 4>(g, p, lds, cus, thr2, pairbuf, scale, gt, st)          \
+                 : launch_bp_as<T, TA, MEM, 1>(g, p, lds, cus, thr2, pairbuf, scale, gt, st))
     return mem == 1 ? RTE_BP(1) : mem == 2 ? RTE_BP(2) : RTE_BP(0);
 #undef RTE_BP
 }

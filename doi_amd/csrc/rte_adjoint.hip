@@ -437,7 +437,8 @@ __global__ __launch_bounds__(1024) void k_backproject_sym(GridDev<T> g, BpPlan p
         // the block's next unit (in a fixed order where the accumulator leaves no room for a counter)
         if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
         const unsigned run = __builtin_amdgcn_readfirstlane(own);
-        const int u = (int)((blockIdx.x + run * (unsigned)p.rot) % gridDim.x + gridDim.x * run);
+        const unsigned b = p.rot ? (blockIdx.x + run * (unsigned)p.rot) % gridDim.x : blockIdx.x;
+        const int u = (int)(b + gridDim.x * run);
         if (gridDim.x * run >= (unsigned)p.nunits) break;
         if (u >= p.nunits) continue;
         const int slab = u & 3, f = (u >> 2) % p.nD + p.nD - 1, first = (u >> 2) / p.nD * M;

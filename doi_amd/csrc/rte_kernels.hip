@@ -378,13 +378,19 @@ __global__ __launch_bounds__(256) void k_to_zpow(int N, const SolveDev<T, TA> *_
 // MEM 0: mu_t from memory; 1: from LDS, the map followed by what the padded voxels
 // of the last bricks reach; 2: from LDS without that tail.  0 and 2 clamp the
 // index of each read (a padded voxel's path; its entry is 0 whatever is read).
-// grid = at most the resident blocks; unit u (translation group, D, SG of the source
-// brick's 64 voxels) belongs to block u mod grid, whose waves share its units.
+// Sources beyond the grid in all M pairs, and rows without a coupled pair, are not marched
+// (150x140x1 50 -> 14 ms, 1x1x1000 3.9 -> 0.33; pair by pair 47 and 1.6).
+// grid = at most the resident blocks; of the units (translation group, D, SG of the source
+// brick's 64 voxels) a block takes one of each run of gridDim.x, its waves share them; which
+// one moves on by rot from run to run where a brick's sources are not all in the grid.
 // ---------------------------------------------------------------------------
 struct KtabPlan {
     int py, pz;       // pitches of y and z in the map read (elements)
     int last;         // largest index of the map read
     int nD, nunits;
+    int rot;          // what a block's unit moves on by from run to run
+    int ragged;       // the last bricks reach beyond the grid
+    int cut;          // a coupling threshold; 2: the table holds zeros
     int next;         // where in LDS the block's unit counter lies (bytes), -1: no room
 };
 
@@ -418,12 +424,20 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
     for (int own = tid / kWave;; own += THREADS / kWave) {
         // the block's next unit (in a fixed order where its map leaves no room for a counter)
         if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
-        const int u = blockIdx.x + gridDim.x * __builtin_amdgcn_readfirstlane(own);
-        if (u >= p.nunits) break;
+        const unsigned run = __builtin_amdgcn_readfirstlane(own);
+        const unsigned b = p.rot ? (blockIdx.x + run * (unsigned)p.rot) % gridDim.x : blockIdx.x;
+        const int u = (int)(b + gridDim.x * run);
+        if (gridDim.x * run >= (unsigned)p.nunits) break;
+        if (u >= p.nunits) continue;
         const int slab = u % NS, f = (u / NS) % p.nD + p.nD - 1, first = (u / NS) / p.nD * M;
         const int Dx = f % ex - (g.bx - 1), Dy = (f / ex) % ey - (g.by - 1), Dz = f / (ex * ey) - (g.bz - 1);
         const int cx = g.bx - abs(Dx), cy = g.by - abs(Dy), cnt = cx * cy * (g.bz - abs(Dz));
         if (first >= cnt) continue;
+        if (p.cut == 2) {  // out, if the bricks' nearest voxels are not coupled (r^2 and thr2 are rounded)
+            const T nx = T(max(0, kBrick * abs(Dx) - 3)) * g.dx, ny = T(max(0, kBrick * abs(Dy) - 3)) * g.dy,
+                    nz = T(max(0, kBrick * abs(Dz) - 3)) * g.dz;
+            if (sum_squares(nx, ny, nz) > thr2 * T(1.0001)) continue;
+        }
         const bool mirror = (Dx | Dy | Dz) != 0;
         // the M source bricks (the last one again where there are fewer): voxel (0,0,0) of each
         int bx0[M], by0[M], bz0[M];
@@ -434,15 +448,49 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
             by0[m] = ((t / cx) % cy + max(0, -Dy)) * kBrick;
             bz0[m] = (t / (cx * cy) + max(0, -Dz)) * kBrick;
         }
+        // bit i: source i is in the grid in some of them (the lowest on each axis); bit 31: a row's
+        // pairs may all be uncoupled
+        unsigned src = (1u << SG) - 1;
+        if (p.ragged) {
+            int lo[3] = {bx0[0], by0[0], bz0[0]};
+#pragma unroll
+            for (int m = 1; m < M; ++m) {
+                lo[0] = min(lo[0], bx0[m]);
+                lo[1] = min(lo[1], by0[m]);
+                lo[2] = min(lo[2], bz0[m]);
+            }
+#pragma unroll
+            for (int i = 0; i < SG; ++i) {
+                const int j = slab * SG + i;
+                if (lo[0] + (j & 3) >= g.nx || lo[1] + ((j >> 2) & 3) >= g.ny || lo[2] + (j >> 4) >= g.nz) src &= ~(1u << i);
+            }
+        }
+        if (p.cut) src |= 0x80000000u;
         T mir[M][SG];
 #pragma unroll
         for (int i = 0; i < SG; ++i) {
             const int j = slab * SG + i, sx = j & 3, sy = (j >> 2) & 3, sz = j >> 4;
+            if (!(src >> i & 1)) {
+#pragma unroll
+                for (int m = 0; m < M; ++m) mir[m][i] = T(0);
+                continue;
+            }
             const int ix = Dx * kBrick + lx - sx, iy = Dy * kBrick + ly - sy, iz = Dz * kBrick + lz - sz;
             const T ddx = T(ix) * g.dx, ddy = T(iy) * g.dy, ddz = T(iz) * g.dz;
             const T r2 = sum_squares(ddx, ddy, ddz);
             const bool self = (ix == 0) && (iy == 0) && (iz == 0);
             const bool use = !self && r2 < thr2;
+            if (src >> 31 && !__any(use)) {  // no lane's pair is coupled
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const int x = bx0[m] + sx, y = by0[m] + sy, z = bz0[m] + sz;
+                    const int bd = (bx0[m] / kBrick + Dx) + g.bx * ((by0[m] / kBrick + Dy) + g.by * (bz0[m] / kBrick + Dz));
+                    mir[m][i] = T(0);
+                    if (x < g.nx && y < g.ny && z < g.nz && first + m < cnt)
+                        ktab[(size_t)(x + g.nx * y + nxy * z) * g.npad + bd * kWave + lane] = T(0);
+                }
+                continue;
+            }
             const T r = sqrt(self ? T(1) : r2);
             // march_tau for M starting voxels
             const int n0 = abs(ix), n1 = abs(iy), n2 = abs(iz);
@@ -1349,6 +1397,8 @@ static hipError_t launch_ktab_as(const GridDev<T> &g, KtabPlan p, size_t lds, in
     constexpr int waves = THREADS / kWave;
     p.nunits = p.nD * ((g.nblk + M - 1) / M) * (kWave / SG);
     const int blocks = min((p.nunits + waves - 1) / waves, cus * (1024 / THREADS));
+    p.ragged = g.nx % kBrick || g.ny % kBrick || g.nz % kBrick;
+    p.rot = (g.ny % kBrick || g.nz % kBrick) ? (int)(0.618 * blocks) | 1 : 0;
     hipLaunchKernelGGL((k_ktab<T, MEM, M, SG, THREADS>), dim3(blocks), dim3(THREADS), lds, st, g, p, thr2, mut, ktab);
     return hipGetLastError();
 }
@@ -1385,6 +1435,25 @@ hipError_t launch_ktab(const GridDev<T> &g, T thr2, const T *mut, T *ktab, hipSt
         lds = 16;
     }
     p.nD = ((2 * g.bx - 1) * (2 * g.by - 1) * (2 * g.bz - 1) + 1) / 2;
+    // Where a threshold leaves more than half of the brick pairs of a table of 32 MB and more
+    // uncoupled, zeros are streamed first and these pairs left out: their rows of 32 and 256 bytes
+    // are written at 1.3 TB/s, a stream at 4 (ms at a threshold of 4.7 voxels, rows / stream and the
+    // rest: 24^3 0.41 / 0.19, 33^3 4.0 / 1.7, 36^3 5.4 / 2.0; 12^3 0.021 / 0.028)
+    double near = 0.0;
+    for (int Dz = 0; Dz < g.bz; ++Dz)
+        for (int Dy = 0; Dy < g.by; ++Dy)
+            for (int Dx = 0; Dx < g.bx; ++Dx) {
+                const double x = max(0, kBrick * Dx - 3) * (double)g.dx, y = max(0, kBrick * Dy - 3) * (double)g.dy,
+                             z = max(0, kBrick * Dz - 3) * (double)g.dz;
+                if (x * x + y * y + z * z <= (double)thr2)
+                    near += (Dx ? 2.0 : 1.0) * (Dy ? 2.0 : 1.0) * (Dz ? 2.0 : 1.0) * (g.bx - Dx) * (g.by - Dy) * (g.bz - Dz);
+            }
+    const double bxl = g.bx * (double)kBrick * g.dx, byl = g.by * (double)kBrick * g.dy, bzl = g.bz * (double)kBrick * g.dz;
+    p.cut = bxl * bxl + byl * byl + bzl * bzl < (double)thr2 ? 0 : near < 0.5 * g.nblk * (double)g.nblk && (size_t)g.N * g.npad * sizeof(T) >= 32u << 20 ? 2 : 1;
+    if (p.cut == 2) {
+        const hipError_t ez = launch_fill<double>(reinterpret_cast<double *>(ktab), (size_t)g.N * g.npad * sizeof(T) / 8, 0.0, st);
+        if (ez != hipSuccess) return ez;
+    }
     // 7 translations and 8 sources per unit (FP64: 8 and 4, at half the waves) -- the most
     // that 1024 threads hold without scratch -- while that leaves the chip's waves several
     // units, else 4 and 4 (more, shorter units).  Either way in ms: 12^3 0.036 / 0.028,

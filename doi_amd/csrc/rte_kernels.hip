@@ -394,7 +394,8 @@ struct KtabPlan {
     int next;         // where in LDS the block's unit counter lies (bytes), -1: no room
 };
 
-template <typename T, int MEM, int M, int SG, int THREADS>
+// PART: a ragged grid or a coupling threshold (without either the checks cost 2 us at 8^3)
+template <typename T, int MEM, int M, int SG, int THREADS, bool PART>
 __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T thr2, const T *__restrict__ mut,
                                                   T *__restrict__ ktab)
 {
@@ -425,7 +426,7 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
         // the block's next unit (in a fixed order where its map leaves no room for a counter)
         if (p.next >= 0 && lane == 0) own = atomicAdd(next, 1);
         const unsigned run = __builtin_amdgcn_readfirstlane(own);
-        const unsigned b = p.rot ? (blockIdx.x + run * (unsigned)p.rot) % gridDim.x : blockIdx.x;
+        const unsigned b = PART && p.rot ? (blockIdx.x + run * (unsigned)p.rot) % gridDim.x : blockIdx.x;
         const int u = (int)(b + gridDim.x * run);
         if (gridDim.x * run >= (unsigned)p.nunits) break;
         if (u >= p.nunits) continue;
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
         const int Dx = f % ex - (g.bx - 1), Dy = (f / ex) % ey - (g.by - 1), Dz = f / (ex * ey) - (g.bz - 1);
         const int cx = g.bx - abs(Dx), cy = g.by - abs(Dy), cnt = cx * cy * (g.bz - abs(Dz));
         if (first >= cnt) continue;
-        if (p.cut == 2) {  // out, if the bricks' nearest voxels are not coupled (r^2 and thr2 are rounded)
+        if (PART && p.cut == 2) {  // out, if the bricks' nearest voxels are not coupled (r^2 and thr2 are rounded)
             const T nx = T(max(0, kBrick * abs(Dx) - 3)) * g.dx, ny = T(max(0, kBrick * abs(Dy) - 3)) * g.dy,
                     nz = T(max(0, kBrick * abs(Dz) - 3)) * g.dz;
             if (sum_squares(nx, ny, nz) > thr2 * T(1.0001)) continue;
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
         // bit i: source i is in the grid in some of them (the lowest on each axis); bit 31: a row's
         // pairs may all be uncoupled
         unsigned src = (1u << SG) - 1;
-        if (p.ragged) {
+        if (PART && p.ragged) {
             int lo[3] = {bx0[0], by0[0], bz0[0]};
 #pragma unroll
             for (int m = 1; m < M; ++m) {
@@ -465,12 +466,12 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
                 if (lo[0] + (j & 3) >= g.nx || lo[1] + ((j >> 2) & 3) >= g.ny || lo[2] + (j >> 4) >= g.nz) src &= ~(1u << i);
             }
         }
-        if (p.cut) src |= 0x80000000u;
+        if (PART && p.cut) src |= 0x80000000u;
         T mir[M][SG];
 #pragma unroll
         for (int i = 0; i < SG; ++i) {
             const int j = slab * SG + i, sx = j & 3, sy = (j >> 2) & 3, sz = j >> 4;
-            if (!(src >> i & 1)) {
+            if (PART && !(src >> i & 1)) {
 #pragma unroll
                 for (int m = 0; m < M; ++m) mir[m][i] = T(0);
                 continue;
@@ -480,7 +481,7 @@ __global__ __launch_bounds__(THREADS) void k_ktab(GridDev<T> g, KtabPlan p, T th
             const T r2 = sum_squares(ddx, ddy, ddz);
             const bool self = (ix == 0) && (iy == 0) && (iz == 0);
             const bool use = !self && r2 < thr2;
-            if (src >> 31 && !__any(use)) {  // no lane's pair is coupled
+            if (PART && src >> 31 && !__any(use)) {  // no lane's pair is coupled
 #pragma unroll
                 for (int m = 0; m < M; ++m) {
                     const int x = bx0[m] + sx, y = by0[m] + sy, z = bz0[m] + sz;
@@ -1385,21 +1386,20 @@ hipError_t device_limits(DevLimits *out)
     return hipSuccess;
 }
 
-template <typename T, int MEM, int M, int SG, int THREADS>
+template <typename T, int MEM, int M, int SG, int THREADS, bool PART>
 static hipError_t launch_ktab_as(const GridDev<T> &g, KtabPlan p, size_t lds, int cus, T thr2, const T *mut, T *ktab,
                                  hipStream_t st)
 {
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ktab<T, MEM, M, SG, THREADS>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ktab<T, MEM, M, SG, THREADS, PART>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     constexpr int waves = THREADS / kWave;
     p.nunits = p.nD * ((g.nblk + M - 1) / M) * (kWave / SG);
     const int blocks = min((p.nunits + waves - 1) / waves, cus * (1024 / THREADS));
-    p.ragged = g.nx % kBrick || g.ny % kBrick || g.nz % kBrick;
     p.rot = (g.ny % kBrick || g.nz % kBrick) ? (int)(0.618 * blocks) | 1 : 0;
-    hipLaunchKernelGGL((k_ktab<T, MEM, M, SG, THREADS>), dim3(blocks), dim3(THREADS), lds, st, g, p, thr2, mut, ktab);
+    hipLaunchKernelGGL((k_ktab<T, MEM, M, SG, THREADS, PART>), dim3(blocks), dim3(THREADS), lds, st, g, p, thr2, mut, ktab);
     return hipGetLastError();
 }
 
@@ -1454,16 +1454,19 @@ hipError_t launch_ktab(const GridDev<T> &g, T thr2, const T *mut, T *ktab, hipSt
         const hipError_t ez = launch_fill<double>(reinterpret_cast<double *>(ktab), (size_t)g.N * g.npad * sizeof(T) / 8, 0.0, st);
         if (ez != hipSuccess) return ez;
     }
+    p.ragged = g.nx % kBrick || g.ny % kBrick || g.nz % kBrick;
     // 7 translations and 8 sources per unit (FP64: 8 and 4, at half the waves) -- the most
     // that 1024 threads hold without scratch -- while that leaves the chip's waves several
     // units, else 4 and 4 (more, shorter units).  Either way in ms: 12^3 0.036 / 0.028,
     // 16^3 0.079 / 0.078, 18^3 0.197 / 0.264, 20^3 0.192 / 0.266, 32^3 3.2 / 3.7
     const bool wide = (long long)g.nblk * (g.nblk + 1) / 2 >= 16LL * cus;
     constexpr bool f32 = sizeof(T) == 4;
-#define RTE_KTAB(MEM)                                                                                           \
-    (wide ? launch_ktab_as<T, MEM, f32 ? 7 : 8, f32 ? 8 : 4, f32 ? 1024 : 512>(g, p, lds, cus, thr2, mut, ktab, st) \
-          : launch_ktab_as<T, MEM, 4, 4, 256>(g, p, lds, cus, thr2, mut, ktab, st))
+#define RTE_KTAB_AS(MEM, PART)                                                                                          \
+    (wide ? launch_ktab_as<T, MEM, f32 ? 7 : 8, f32 ? 8 : 4, f32 ? 1024 : 512, PART>(g, p, lds, cus, thr2, mut, ktab, st) \
+          : launch_ktab_as<T, MEM, 4, 4, 256, PART>(g, p, lds, cus, thr2, mut, ktab, st))
+#define RTE_KTAB(MEM) (p.ragged || p.cut ? RTE_KTAB_AS(MEM, true) : RTE_KTAB_AS(MEM, false))
     return mem == 1 ? RTE_KTAB(1) : mem == 2 ? RTE_KTAB(2) : RTE_KTAB(0);
+#undef RTE_KTAB_AS
 #undef RTE_KTAB
 }
 

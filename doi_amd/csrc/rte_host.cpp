@@ -472,7 +472,8 @@ struct rte_medium {
     double ktab_f_thr = -1, ktab_d_thr = -1;
     DevBuf kexp;  // exponents of ktab_f, if kexp_ok
     bool kexp_ok = false;
-    OptRange range;
+    OptRange range;  // if range_ok (even_medium looks at it, on large grids only)
+    bool range_ok = false;
 };
 
 static int set_device(rte_ctx *ctx)
@@ -718,7 +719,6 @@ extern "C" int rte_medium_create(rte_ctx *ctx, const rte_grid *grid, const rte_o
     const size_t N = (size_t)m->N;
     m->mua_h.assign(optics->mu_a, optics->mu_a + N);
     m->mus_h.assign(optics->mu_s, optics->mu_s + N);
-    m->range = opt_range(optics->mu_a, optics->mu_s, N);
     std::vector<float> mt_f(N), ms_f(N);
     std::vector<double> mt_d(N);
     for (size_t v = 0; v < N; ++v) {
@@ -854,7 +854,8 @@ static int ensure_kexp(rte_medium *m)
 
 // ---- how a grid's propagation runs ------------------------------------------
 // Chunks (of source brick rows) of the matrix-core propagation of a solve alone, and its
-// estimated time in us: rounds of its workgroups over 256 CUs, each one's tiles (a source
+// estimated time in us: rounds of its workgroups over 256 CUs (of the whole chip, whatever
+// device runs it: a solve's bits are not to depend on that), each one's tiles (a source
 // slab, 4.3 us) and its start, and the partial sums' way through memory.
 static double mfma_chunks(const GridDev<float> &g, int K, int *nchunk)
 {
@@ -897,19 +898,31 @@ static bool even_medium(const rte_grid &gr, const OptRange &r, double thr)
 
 // Whether the FP32 cached propagation of a grid runs on the matrix cores (rte_mfma.hip):
 // L = 4 and 5, where a solve alone is to take at most 0.95 of k_prop's time there (2.34
-// and 2.94 ps a pair), which is where no group of solves measured slower.  It depends on
-// the grid, the order and the solve's medium (even) only, so that a solve takes the same
-// kernel, and has the same bits, alone and in any batch.
-static bool use_mfma(int L, const GridDev<float> &g, bool even)
+// and 2.94 ps a pair), which is where no group of solves measured slower (22 grids, cubes
+// of 24 to 36, flat, long and ragged ones, 1 to 16 solves on 1 to 3 media: 1.02 to 1.85
+// times k_prop's speed; closest 35^3 3 beams 13.6 against 13.3 ms a term, 30^3 5 beams 7.5
+// against 6.9).
+static bool mfma_grid(int L, const GridDev<float> &g)
 {
-    if (!even || (L != 4 && L != 5)) return false;
+    if (L != 4 && L != 5) return false;
     int nch = 1;
     return mfma_chunks(g, (L + 1) * (L + 1), &nch) < 0.95 * (L == 4 ? 2.34e-6 : 2.94e-6) * g.N * (double)g.N;
 }
 
+// ... and a solve's: it depends on the grid, the order and the solve's own medium and
+// threshold only, so that a solve takes the same kernel, and has the same bits, alone and
+// in any batch
+static bool medium_on_mfma(rte_medium *m, int L, double thr)
+{
+    if (!mfma_grid(L, make_grid<float>(m->grid))) return false;
+    if (!m->range_ok) m->range = opt_range(m->mua_h.data(), m->mus_h.data(), m->N);
+    m->range_ok = true;
+    return even_medium(m->grid, m->range, thr);
+}
+
 // The chunks of a propagation and the size of its input copy Wp (in T); depends on
-// the grid, order, path and medium only, so that a solve's partial sums, and its bits, are the
-// same alone and in any batch.
+// the grid, the order and whether it runs on the matrix cores (on) only, so that a solve's
+// partial sums, and its bits, are the same alone and in any batch.
 struct PropShape {
     bool mfma = false;
     int nch = 1, clen = 0;
@@ -917,12 +930,12 @@ struct PropShape {
 };
 
 template <typename T>
-static PropShape prop_shape(const GridDev<T> &g, int L, int path, bool cplx, bool even)
+static PropShape prop_shape(const GridDev<T> &g, int L, bool on)
 {
     PropShape s;
     const int K = (L + 1) * (L + 1);
     if constexpr (sizeof(T) == 4) {
-        if (path == RTE_PATH_CACHED && !cplx && use_mfma(L, g, even)) {
+        if (on) {
             s.mfma = true;
             mfma_chunks(g, K, &s.nch);
             s.wp = mfma_wp_bytes(L, g) / sizeof(T);
@@ -1152,7 +1165,8 @@ static int run_batch(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_b
         for (int i = 0; i < nb; ++i)
             if ((rc = ensure_ktab<T>(media[i], thr))) return rc;
 
-    const PropShape sh = prop_shape<T>(g, L, path, kim != nullptr, even_medium(grid, media[0]->range, thr));
+    const bool on = sizeof(T) == 4 && path == RTE_PATH_CACHED && !kim && medium_on_mfma(media[0], L, thr);
+    const PropShape sh = prop_shape<T>(g, L, on);
     const int nch = sh.nch;
     PropArgs<T> pa;
     std::shared_ptr<DevBuf> zt;
@@ -1516,12 +1530,6 @@ static int check_params(const rte_params *p)
     return RTE_OK;
 }
 
-static bool on_matrix_cores(const rte_grid &grid, const rte_params &p, const OptRange &r)
-{
-    return p.precision != RTE_PREC_FP64 && p.path_mode == RTE_PATH_CACHED &&
-           use_mfma(p.L, make_grid<float>(grid), even_medium(grid, r, p.prop_thresh));
-}
-
 static int solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, const rte_beam *beams,
                         const rte_params *params, double *exitance, double *reflectance, rte_stats *stats)
 {
@@ -1555,7 +1563,9 @@ extern "C" int rte_solve_images(rte_ctx *ctx, int nb, rte_medium *const *media, 
     if ((rc = set_device(ctx))) return rc;
     // solves that the matrix cores take and solves that they do not are batches of their own
     std::vector<int> on, off;
-    for (int i = 0; i < nb; ++i) (on_matrix_cores(media[i]->grid, *params, media[i]->range) ? on : off).push_back(i);
+    if (params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
+        mfma_grid(params->L, make_grid<float>(media[0]->grid)))
+        for (int i = 0; i < nb; ++i) (medium_on_mfma(media[i], params->L, params->prop_thresh) ? on : off).push_back(i);
     if (on.empty() || off.empty()) return solve_images(ctx, nb, media, beams, params, exitance, reflectance, stats);
     const size_t P = (size_t)media[0]->grid.nx * media[0]->grid.ny;
     double gpu_ms = 0.0;
@@ -1821,12 +1831,13 @@ extern "C" int rte_solve(rte_ctx *ctx, const rte_grid *grid, const rte_optics *o
     return rc;
 }
 
-extern "C" int rte_on_matrix_cores(const rte_medium *m, const rte_params *params)
+extern "C" int rte_on_matrix_cores(rte_medium *m, const rte_params *params)
 {
     if (!m) return fail(RTE_E_ARG, "rte_on_matrix_cores: NULL medium");
     int rc;
     if ((rc = check_params(params))) return rc;
-    return on_matrix_cores(m->grid, *params, m->range);
+    return params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
+           medium_on_mfma(m, params->L, params->prop_thresh);
 }
 
 // device memory of one solve of a shape; on: it propagates on the matrix cores
@@ -1835,7 +1846,7 @@ static long long solve_bytes(const rte_grid &grid, const rte_params &p, int path
     const GridDev<float> g = make_grid<float>(grid);
     const long long K = (p.L + 1) * (p.L + 1), N = g.N;
     const long long es = p.precision == RTE_PREC_FP64 ? 8 : 4;
-    const PropShape sh = prop_shape<float>(g, p.L, on ? RTE_PATH_CACHED : RTE_PATH_MARCH, false, true);
+    const PropShape sh = prop_shape<float>(g, p.L, on);
     long long bytes = N * 8 * 3 + N * 4 * 2;                    // maps
     bytes += N * K * es * (1 + sh.nch) + (long long)sh.wp * es;  // W, partials, the propagation's copy of W
     bytes += (long long)grid.nx * grid.ny * kPixBufs * 8 + 64;   // pixel buffers
@@ -1910,8 +1921,7 @@ struct AdjointRun {
         clen = (N + nch0 - 1) / nch0;
         nch = (N + clen - 1) / clen;
         F = (size_t)N * K;
-        // the forward series'
-        const PropShape sh = prop_shape<T>(g, L, RTE_PATH_CACHED, false, even_medium(grid, m->range, thr));
+        const PropShape sh = prop_shape<T>(g, L, sizeof(T) == 4 && medium_on_mfma(m, L, thr));  // the forward series'
         if (sh.mfma && (rc = ensure_kexp(m))) return rc;
         HIP_TRY(dW.alloc(F * sizeof(T)));
         HIP_TRY(dWp.alloc(sh.wp * sizeof(T)));
@@ -2522,7 +2532,7 @@ static int propagate_impl(rte_ctx *ctx, rte_medium *m, int L, double prop_thresh
     int rc;
     if ((rc = get_moments(ctx, L, dx, dy, dz, &mom))) return rc;
     if (path == RTE_PATH_CACHED && (rc = ensure_ktab<T>(m, thr))) return rc;
-    const PropShape sh = prop_shape<T>(g, L, path, false, even_medium(grid, m->range, thr));
+    const PropShape sh = prop_shape<T>(g, L, sizeof(T) == 4 && path == RTE_PATH_CACHED && medium_on_mfma(m, L, thr));
     const int nch = sh.nch;
     PropArgs<T> pa;
     std::shared_ptr<DevBuf> zt;
@@ -3044,7 +3054,7 @@ struct Bucket : BucketBase {
         max_terms = p.max_terms > 0 ? p.max_terms : 1000;
         slot_bytes = solve_bytes(grid, p, p.path_mode, on);
         // the same source chunking as rte_solve_media
-        sh = prop_shape<T>(g, L, p.path_mode, false, on);
+        sh = prop_shape<T>(g, L, on);
         sc = make_scales(L);
         std::memset(&ca, 0, sizeof ca);
         ca.g = g;
@@ -3610,7 +3620,9 @@ extern "C" int rte_submit(rte_server *S, const rte_grid *grid, const rte_optics 
     r->g = optics->g;
     r->beam = *beam;
     r->params = *params;
-    r->on = on_matrix_cores(*grid, *params, opt_range(optics->mu_a, optics->mu_s, N));
+    r->on = params->precision != RTE_PREC_FP64 && params->path_mode == RTE_PATH_CACHED &&
+            mfma_grid(params->L, make_grid<float>(*grid)) &&
+            even_medium(*grid, opt_range(optics->mu_a, optics->mu_s, N), params->prop_thresh);
     r->key = bucket_key(*grid, *params, r->on);
     r->footprint = solve_bytes(*grid, *params, params->path_mode, r->on);
     std::lock_guard<std::mutex> lk(S->mu);

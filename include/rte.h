@@ -171,7 +171,7 @@ int rte_medium_destroy(rte_medium *m);
 int rte_medium_reset_cache(rte_medium *m);
 /* 1 if solves on this medium propagate on the matrix cores, 0 if not (see RTE_PREC_FP32; it
  * depends on the medium and params alone, not on what shares a call with the solve), or RTE_E* */
-int rte_on_matrix_cores(const rte_medium *m, const rte_params *params);
+int rte_on_matrix_cores(rte_medium *m, const rte_params *params);
 /* bytes of device memory a solve of this shape needs (admission by HBM footprint); on the
  * matrix cores 1/64 of the path table and its partial sums come on top (a server counts
  * them), and a table of displacements that all solves of the grid share */

@@ -10,17 +10,18 @@
 //   T(d, s, c)  = kf(d + t_c, s + t_c) P(d, c)            the only per-pair work left on the VALU
 //   acc(j, c)  += sum_s Z_j(d-s) T(d, s, c)              one product per destination d: K x 16 c
 // Z and W, and then Z and T, go through v_mfma_f32_16x16x32_f16 as two FP16 pieces each
-// (x = h + l to 22 bits, products hh + hl + lh, sums in FP32); powers of two keep every
-// piece in range and are taken out of each tile's sums: for W the largest of its source
-// slab and right-hand side, for T the largest path-table entry of the source slab and
-// destination (k_kexp).  Error against FP64 at 24^3, L = 5: rms 2.18e-6, 2.24e-6 on the
-// FP32 vector pipe; most of both is the path table's.
+// (x = h + l, Z and W to 24 bits, T to 22; products hh + hl + lh, sums in FP32); powers of two
+// keep every piece in range and are taken out of each tile's sums: for W the largest of its
+// source slab and right-hand side, for T the largest path-table entry of the source slab and
+// destination (k_kexp).  Media where these leave a contribution fewer bits than FP32 run
+// k_prop (even_medium).  Error of 32^3, L = 5 solves against FP64 2.8e-7 to 4.4e-7, on the FP32
+// vector pipe 6.2e-7 to 6.4e-7.
 //
 // Measured per term at 32^3 (k_prop, all VALU, whose FMAs run at 94 % of the pipe's rate ->
-// this): L = 5 one solve 3.16 -> 2.15 ms, 5 beams 9.3 -> 7.2, 15 on 3 media 26.6 -> 16.4;
-// L = 4 2.55 -> 1.81, 7.4 -> 6.0, 19.0 -> 13.5.  Bound of the last L = 5 launch (16.7 ms for 16):
-// issue of a SIMD's two waves (VALU 37 %, MFMA 24 % of the clocks, mostly one after the
-// other) and LDS (45 %); the rest is waits at the tile's two barriers.
+// this): L = 5 one solve 3.28 -> 2.10 ms, 5 beams 9.4 -> 7.3, 15 on 3 media 27.5 -> 16.6;
+// L = 4 2.71 -> 1.80, 7.5 -> 6.1, 19.7 -> 13.9.  Bound in the benchmark's launches: issue of a
+// SIMD's two waves (VALU 40 %, MFMA 28 % of the clocks, mostly one after the other) and LDS
+// (48 %, 9 % bank conflicts); the rest is waits at the tile's two barriers.
 #include "rte_device.hpp"
 
 namespace rte {
